@@ -187,7 +187,9 @@ int vrn_timing_report(vrn_ctx *ctx, char *names, int name_len, int64_t *counts, 
  * x sweep: rows_per_wave whole rows per wavefront, or, with xseg > 1, one of
  * xseg segments of a row per wavefront (then rows_per_wave must be 1);
  * y / z sweeps: seg_len interior cells per marching segment.  vrn_create
- * chooses a partition for the grid; vrn_get_partition reads it back. */
+ * chooses a partition for the grid, with a segment for each march and form
+ * (from 1 cell on small grids); vrn_get_partition reads it back, as seg_len
+ * the FP64 y march's and at least 8, the least that can be set. */
 int vrn_set_partition(vrn_ctx *ctx, int rows_per_wave, int xseg, int seg_len);
 int vrn_get_partition(vrn_ctx *ctx, int *rows_per_wave, int *xseg, int *seg_len);
 

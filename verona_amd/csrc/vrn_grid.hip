@@ -421,7 +421,7 @@ struct vrn_ctx {
     double dxs[3] = {1, 1, 1};
     // tuning
     int rows_per_wave = 8;
-    int seg_len = 96;
+    int seg_y[2] = {96, 96}, seg_z[2] = {96, 96};  // FP64, FP32 forms
     int xseg = 1;
     // timing
     int timing = 0;  // 0 off, 1 every kernel, 2 the directional sweeps only
@@ -575,11 +575,6 @@ int check_ctx(vrn_ctx *c)
 }  // namespace
 
 // ====================================================================== C ABI
-// Work partition of the sweeps for this grid: enough waves to fill 256 CUs
-// (x sweep: whole rows per wave while rows are plentiful, else segments of
-// one row; y / z sweeps: shorter marching segments when columns are few).
-// The partition changes no arithmetic: every face is solved once and every
-// cell updated once from the same operands.
 // Fill the x faces the last stage-end ghost pass left unfilled, if any.
 static int settle(vrn_ctx *c)
 {
@@ -594,6 +589,57 @@ static int settle(vrn_ctx *c)
     return 0;
 }
 
+// Interior cells per marching segment of one y or z march: L cells along the
+// march, `cols` blocks across it (256 lanes in 3D, 64 in 2D), fp32: the FP32
+// form.  A segment of s cells costs s rows and about two rows of warm-up (two
+// more cells are reconstructed than updated, and the ring is filled).  The
+// registers and the LDS ring let each CU hold 2 blocks of the FP64 march (3 of
+// the FP32 one, 4 times as many in 2D), so with b blocks in all the march
+// takes about (s + 2) f(b) row times, with
+//   f = 0.6   while every SIMD has at most one wave (a second one slows both:
+//             128^3, 32 cells in 256 blocks 152 us, 16 in 512 blocks 139 us),
+//   f = 1.1   while all blocks are resident (2D: 1.0, two full rounds of 16
+//             cells take 185 us at 2048^2 where one of 32 cells takes 173),
+//   beyond that between whole rounds (short marches keep step: 96^3, 8 cells
+//             in 576 blocks 98 us, 6 cells in 768 blocks 81 us) and a steady
+//             stream of blocks with one partly empty round.
+// Measured, fast FP64 form, x-y march: 32^3 24 cells 107 us, 1 cell 17 us;
+// 64^3 24 cells 110 us, 8 cells 45 us, 4 cells 30 us, 1 cell 43 us; 192^3 64
+// cells 493 us, 28 cells 426 us, 16 cells 422 us, 8 cells 442 us; 256^3 96 /
+// 48 / 24 / 8 cells 957 / 945 / 961 / 1051 us; 2D 256^2 24 cells 77 us, 1
+// cell 17 us; 2048^2 32 cells 173 us, 24 cells 188 us, 8 cells 177 us.
+// Segments are evened out (the shortest ones of the same count).
+static int march_segment(int ndim, bool fp32, int L, int cols)
+{
+    const int one = 256 * (ndim == 3 ? 1 : 4);  // blocks at one wave per SIMD
+    const int slots = one * (fp32 ? 3 : 2);
+    int best = L;
+    double least = 1e300;
+    for (int n = 1; n <= L && n <= 65535; n++) {
+        const int s = (L + n - 1) / n;
+        if (n > 1 && (L + n - 2) / (n - 1) == s) continue;  // same segments as n - 1
+        const long b = (long)cols * n, rem = b % slots;
+        double f;
+        if (b <= one)
+            f = 0.6;
+        else if (b <= slots)
+            f = ndim == 3 ? 1.1 : 1.0;
+        else
+            f = 0.5 * ((double)(b / slots) + (rem == 0 ? 0.0 : (rem <= one ? 0.6 : 1.0)) + 0.85 * b / slots + 0.3);
+        const double t = (s + 2) * f;
+        if (t < least) {
+            least = t;
+            best = s;
+        }
+    }
+    return best;
+}
+
+// Work partition of the sweeps for this grid: enough waves to fill 256 CUs
+// (x sweep: whole rows per wave while rows are plentiful, else segments of
+// one row; y / z sweeps: march_segment of each march).
+// The partition changes no arithmetic: every face is solved once and every
+// cell updated once from the same operands.
 static void partition_sweeps(vrn_ctx *c)
 {
     const int Nxi = c->G.NX - 6, Nyi = c->G.NY - 6, Nzi = c->ndim == 3 ? c->G.NZ - 6 : 1;
@@ -608,10 +654,11 @@ static void partition_sweeps(vrn_ctx *c)
         if (c->xseg < 1) c->xseg = 1;
         if (c->xseg > 1) c->rows_per_wave = 1;
     }
-    const long colwaves = (long)((Nxi + 63) / 64) * (c->ndim == 3 ? (Nyi < Nzi ? Nyi : Nzi) : 1);
-    const int along = c->ndim == 3 ? (Nyi > Nzi ? Nyi : Nzi) : Nyi;
-    long seg = colwaves * along / 2048;
-    c->seg_len = (int)(seg < 24 ? 24 : (seg > 96 ? 96 : seg));
+    for (int f = 0; f < 2; f++) {
+        const int nxb = (Nxi + 63) / 64;
+        c->seg_y[f] = march_segment(c->ndim, f == 1, Nyi, nxb * (c->ndim == 3 ? (Nzi + 3) / 4 : 1));
+        c->seg_z[f] = march_segment(c->ndim, f == 1, Nzi, nxb * ((Nyi + 3) / 4));
+    }
 }
 
 extern "C" {
@@ -1067,7 +1114,9 @@ int vrn_step(vrn_ctx *c, const vrn_step_params *p, double *dt_used)
     a.n_iter = p->n_iter;
     a.dt_fixed = p->dt;
     a.dt_dev = cflm ? 1 : 0;
-    a.seg_len = c->seg_len;
+    const int sf = p->precision == VRN_PREC_FP32 ? 1 : 0;
+    a.seg_y = c->seg_y[sf];
+    a.seg_z = c->seg_z[sf];
     a.rows_per_wave = c->rows_per_wave;
     a.xseg = c->xseg;
     a.fuse_xy = c->fuse_xy;
@@ -1155,7 +1204,7 @@ int vrn_set_partition(vrn_ctx *c, int rows_per_wave, int xseg, int seg_len)
         return fail(VRN_E_ARG, "row segments shorter than 32 cells (nx %d, xseg %d)", Nxi, xseg);
     c->rows_per_wave = rows_per_wave;
     c->xseg = xseg;
-    c->seg_len = seg_len;
+    for (int f = 0; f < 2; f++) c->seg_y[f] = c->seg_z[f] = seg_len;
     return 0;
 }
 
@@ -1171,7 +1220,9 @@ int vrn_get_partition(vrn_ctx *c, int *rows_per_wave, int *xseg, int *seg_len)
     if (int r = check_ctx(c)) return r;
     if (rows_per_wave) *rows_per_wave = c->rows_per_wave;
     if (xseg) *xseg = c->xseg;
-    if (seg_len) *seg_len = c->seg_len;
+    // while each march has its own: the FP64 y march's, at least the least that
+    // vrn_set_partition takes
+    if (seg_len) *seg_len = std::max(8, c->seg_y[0]);
     return 0;
 }
 

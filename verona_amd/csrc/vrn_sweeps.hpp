@@ -677,7 +677,8 @@ void launch_stage(hipStream_t s, const SweepArgs &a, const double dxs[3], void (
             SweepArgs ay = a;
             ay.dx_dim = dxs[1];
             ay.dx_x = dxs[0];
-            int nseg = (G.NY - 6 + a.seg_len - 1) / a.seg_len;
+            ay.seg_len = a.seg_y;
+            int nseg = (G.NY - 6 + a.seg_y - 1) / a.seg_y;
             timer(tctx, 10, 0);
             hipLaunchKernelGGL((k_march<5, 1, R, REC, RIEM, false, true>), dim3(nxb, (G.NZ - 6 + 3) / 4, nseg),
                                dim3(256), 0, s, ay);
@@ -696,7 +697,8 @@ void launch_stage(hipStream_t s, const SweepArgs &a, const double dxs[3], void (
         if (!fxy) {
             SweepArgs ay = a;
             ay.dx_dim = dxs[1];
-            int nseg = (G.NY - 6 + a.seg_len - 1) / a.seg_len;
+            ay.seg_len = a.seg_y;
+            int nseg = (G.NY - 6 + a.seg_y - 1) / a.seg_y;
             timer(tctx, 1, 0);
             hipLaunchKernelGGL((k_march<5, 1, R, REC, RIEM, false>), dim3(nxb, (G.NZ - 6 + 3) / 4, nseg), dim3(256), 0, s, ay);
             timer(tctx, 1, 1);
@@ -704,7 +706,8 @@ void launch_stage(hipStream_t s, const SweepArgs &a, const double dxs[3], void (
         {
             SweepArgs az = a;
             az.dx_dim = dxs[2];
-            int nseg = (G.NZ - 6 + a.seg_len - 1) / a.seg_len;
+            az.seg_len = a.seg_z;
+            int nseg = (G.NZ - 6 + a.seg_z - 1) / a.seg_z;
             timer(tctx, 2, 0);
             hipLaunchKernelGGL((k_march<5, 2, R, REC, RIEM, true>), dim3(nxb, (G.NY - 6 + 3) / 4, nseg), dim3(256), 0, s, az);
             timer(tctx, 2, 1);
@@ -717,7 +720,8 @@ void launch_stage(hipStream_t s, const SweepArgs &a, const double dxs[3], void (
     } else {
         SweepArgs ay = a;
         ay.dx_dim = dxs[1];
-        int nseg = (G.NY - 6 + a.seg_len - 1) / a.seg_len;
+        ay.seg_len = a.seg_y;
+        int nseg = (G.NY - 6 + a.seg_y - 1) / a.seg_y;
 #if defined(VRN_FAST)
         // fast FP64 form: the y sweep is the last sweep (RK combination,
         // closed-form 4x4 Newton, Limit and rate inside the march); same
