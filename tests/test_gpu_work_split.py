@@ -36,3 +36,22 @@ def test_automatic_march_segments(shape, form):
             outs.append((dev.download("P"), dev.download("U")))
     for a, b in zip(*outs):
         assert np.array_equal(a, b, equal_nan=True)
+
+
+@pytest.mark.parametrize("n", [1, 3, 63, 64, 65, 129, 8191, 8193, 65536])
+def test_training_gradient_of_any_batch(n):
+    """Slices of the batch that are empty, partly filled or longer than the
+    samples a block holds at a time.  FP32 sums of at most 1024 + 64 terms
+    against 64 bits: 1e-4 of the gradient's norm, as the other gradient test."""
+    import mlp_ref
+    from verona_amd.c2p import Con2PrimBatch, c4_states
+    progress(f"training gradient n={n}")
+    with Con2PrimBatch(1 << 17, G) as cp:
+        X, T, ok = cp.features(*c4_states(1 << 17, seed=9, gamma=G))
+        X, T = X[ok][:n], T[ok][:n]
+        assert len(X) == n
+        params = mlp_ref.he_init(13)
+        loss, g = cp.grad(X, T, params, qat=False, q_ref=0.01)
+    lr, gr = mlp_ref.loss_grad(params, X, T, qat=False, q_ref=0.01)
+    assert abs(loss - lr) <= 1e-4 * lr
+    assert np.linalg.norm(g - gr) <= 1e-4 * np.linalg.norm(gr)

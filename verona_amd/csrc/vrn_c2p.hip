@@ -27,11 +27,9 @@
 // W1, W2, W3 and both hidden layers; FP32: the biases (accumulator
 // initialisation) and accumulation.
 //
-// Training (FP32 VALU): one thread per sample runs forward and backward with
-// the parameters in LDS and caches per-sample activations and deltas; weight
-// gradients are sums over samples, formed by a thread per parameter over a
-// fixed slice of the batch and then a fixed-order sum over slices, so the
-// result is deterministic; Adam runs one thread per parameter.
+// Training (FP32 VALU) is one launch a step (k_train_step).  Weight gradients
+// are sums over samples in a fixed order (64 slices of the batch, then the
+// slices), so the result is deterministic.
 #include "../../include/verona_c2p.h"
 #define VRN_NS vrn_c4
 #include "vrn_physics.hpp"
@@ -44,6 +42,7 @@
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <utility>
 #include <vector>
 
 namespace vrn_c4 {
@@ -693,11 +692,6 @@ __global__ void __launch_bounds__(256) k_infer(long n, const float *__restrict__
 }
 
 // ---------------------------------------------------------------- training
-// Per-sample cache layout (floats): x[8] h1[64] h2[64] dz1[64] dz2[64] dy[2] loss[1]
-constexpr int C_X = 0, C_H1 = 8, C_H2 = C_H1 + NH, C_DZ1 = C_H2 + NH, C_DZ2 = C_DZ1 + NH,
-              C_DY = C_DZ2 + NH, C_L = C_DY + NOUT, C_STRIDE = 272;
-static_assert(C_L < C_STRIDE, "cache stride");
-
 __device__ __forceinline__ unsigned long long splitmix(unsigned long long x)
 {
     x += 0x9E3779B97F4A7C15ull;
@@ -706,6 +700,24 @@ __device__ __forceinline__ unsigned long long splitmix(unsigned long long x)
     return x ^ (x >> 31);
 }
 
+// Training state after a step: parameters, Adam moments and the gradient
+// sums of the slices (row s: the NPARAM sums and the loss of slice s).  Two
+// of them alternate, so that every block of a step can read the last one.
+constexpr int NSPLIT = 64;
+struct TrainState {
+    float prm[NPARAM], m[NPARAM], v[NPARAM];
+    float part[NSPLIT][NPARAM + 1];
+};
+
+// The Adam update that is due before a step (its gradient: the slice sums of
+// `in`), none for the first step.
+struct AdamArgs {
+    int due;
+    int nsplit;
+    float lr, b1, b2, eps, bc1, bc2;
+    float *loss_out;
+};
+
 struct TrainArgs {
     const float *X, *T;
     const int *idx;      // valid-sample list (sampling) or NULL (identity)
@@ -713,138 +725,256 @@ struct TrainArgs {
     int B;
     unsigned long long seed;
     int step;
-    const float *prm;
-    float *cache;
+    const TrainState *in;
+    TrainState *out;
+    AdamArgs adam;
     float w1;
     float q_ref;  // > 0: the first output's squared error weighted by 1 + (q / q_ref)^2
     int qat;
 };
 
-__global__ void __launch_bounds__(256) k_train_fwd_bwd(TrainArgs a)
+// Parameter p of this step: the update of `in` by the gradient its slices
+// hold (summed in slice order), written to `out` by the first block.
+__device__ __forceinline__ float due_param(const AdamArgs &a, const TrainState *in, TrainState *out, int p, bool first)
 {
-    __shared__ float w[NPARAM];
-    for (int p = threadIdx.x; p < NPARAM; p += blockDim.x) {
-        float v = a.prm[p];
+    if (!a.due) {
+        const float w = p < NPARAM ? in->prm[p] : 0.0f;
+        if (first && p < NPARAM) {
+            out->prm[p] = w;
+            out->m[p] = in->m[p];
+            out->v[p] = in->v[p];
+        }
+        return w;
+    }
+    float g = 0.0f;
+    if (a.nsplit == NSPLIT) {
+#pragma unroll
+        for (int s = 0; s < NSPLIT; s++) g = g + in->part[s][p];
+    } else {
+        for (int s = 0; s < a.nsplit; s++) g = g + in->part[s][p];
+    }
+    if (p == NPARAM) {
+        if (first && a.loss_out) *a.loss_out = g;
+        return 0.0f;
+    }
+    const float mm = a.b1 * in->m[p] + (1.0f - a.b1) * g;
+    const float vv = a.b2 * in->v[p] + (1.0f - a.b2) * g * g;
+    const float w = in->prm[p] - a.lr * (mm / a.bc1) / (__builtin_sqrtf(vv / a.bc2) + a.eps);
+    if (first) {
+        out->prm[p] = w;
+        out->m[p] = mm;
+        out->v[p] = vv;
+    }
+    return w;
+}
+
+// Value of lane `Q` of the quad (DPP quad_perm broadcast).
+template <int Q> __device__ __forceinline__ float quad_bcast(float v)
+{
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), Q * 0x55, 0xf, 0xf, true));
+}
+// f(0) .. f(NH - 1) with constant arguments
+template <class F, int... K> __device__ __forceinline__ void each_of(F &f, std::integer_sequence<int, K...>)
+{
+    (f(std::integral_constant<int, K>{}), ...);
+}
+template <class F> __device__ __forceinline__ void each_unit(F f) { each_of(f, std::make_integer_sequence<int, NH>{}); }
+
+// One training step in one launch: the Adam update due from the step before,
+// forward and backward of this step's samples, and their gradient sums.
+// Block s owns slice s of the batch (64 slices, each summed in sample order,
+// then the slices in order: the sums do not depend on the launch).  A step
+// is a chain of short dependent parts on 64 CUs, bound by their latencies:
+//  * every block forms the updated parameters itself from the slice sums of
+//    the last launch (99 KB), so that no launch or grid-wide barrier lies
+//    between reduction, update and the next forward pass; the gather of the
+//    first samples is issued before it;
+//  * a sample is four lanes, four hidden units a lane, exchanged by DPP; one
+//    sample a lane uses 2 of the 8 waves that 128 samples fill this way;
+//  * activations and deltas stay in LDS, [feature][sample], and a lane sums
+//    one parameter from rows of it, four samples a read.  Rows are 4 words
+//    past a multiple of 64, so the rows that a wave reads lie in different
+//    banks.
+// 8192 samples a step: 77 us (forward/backward 12.6, sums from an HBM cache
+// of the activations 44.7, reduction 15.5, Adam 4.6) -> 9.3 us.
+constexpr int TS = 128;       // samples at a time
+constexpr int TROW = TS + 4;  // LDS row
+constexpr int R_X = 0, R_H1 = NIN, R_H2 = R_H1 + NH, R_DZ1 = R_H2 + NH, R_DZ2 = R_DZ1 + NH, R_DY = R_DZ2 + NH,
+              R_L = R_DY + NOUT, R_ROWS = R_L + 1;
+constexpr int W2ROW = NH + 4;  // LDS row of W2: the rows of the quad's lanes start in different banks
+
+__global__ void __launch_bounds__(4 * TS) k_train_step(TrainArgs a)
+{
+    __shared__ __attribute__((aligned(16))) float act[R_ROWS * TROW];
+    __shared__ __attribute__((aligned(16))) float w1[NH * NIN], w2[NH * W2ROW], w3[NOUT * NH];
+    __shared__ float b1[NH], b2[NH], b3[NOUT];
+    static_assert(NIN == 4 && NH == 16 && NOUT == 2, "four units a lane");
+    const int tid = threadIdx.x, q = tid & 3, ls = tid >> 2;
+    const int per = (a.B + a.adam.nsplit - 1) / a.adam.nsplit;
+    const int s0 = blockIdx.x * per, s1 = min(a.B, s0 + per);
+
+    float4 xn;
+    float2 tn;
+    auto gather = [&](int s) {
+        xn = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        tn = make_float2(0.0f, 0.0f);
+        if (s < s1) {
+            long id = s;
+            if (a.idx) {
+                const unsigned long long r =
+                    splitmix(a.seed ^ ((unsigned long long)a.step * 0x100000001B3ull + (unsigned long long)s));
+                id = a.idx[(long)(r % (unsigned long long)a.n_idx)];
+            }
+            xn = *reinterpret_cast<const float4 *>(a.X + (long)NIN * id);
+            tn = *reinterpret_cast<const float2 *>(a.T + 2 * id);
+        }
+    };
+    gather(s0 + ls);
+
+    for (int p = tid; p <= NPARAM; p += 4 * TS) {
+        float w = due_param(a.adam, a.in, a.out, p, blockIdx.x == 0);
         // BF16 in inference: W1, W2, W3 (the biases are FP32 accumulator inputs)
         const bool is_w = p < OFF_B1 || (p >= OFF_W2 && p < OFF_B2) || (p >= OFF_W3 && p < OFF_B3);
-        w[p] = (a.qat && is_w) ? bf16_round(v) : v;
+        if (a.qat && is_w) w = bf16_round(w);
+        if (p < OFF_B1) w1[p] = w;
+        else if (p < OFF_W2) b1[p - OFF_B1] = w;
+        else if (p < OFF_B2) w2[(p - OFF_W2) / NH * W2ROW + (p - OFF_W2) % NH] = w;
+        else if (p < OFF_W3) b2[p - OFF_B2] = w;
+        else if (p < OFF_B3) w3[p - OFF_W3] = w;
+        else if (p < NPARAM) b3[p - OFF_B3] = w;
     }
     __syncthreads();
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= a.B) return;
-    long id = s;
-    if (a.idx) {
-        unsigned long long r = splitmix(a.seed ^ ((unsigned long long)a.step * 0x100000001B3ull + (unsigned long long)s));
-        id = a.idx[(long)(r % (unsigned long long)a.n_idx)];
-    }
-    float *c = a.cache + (long)s * C_STRIDE;
-    float x[NIN];
-#pragma unroll
-    for (int k = 0; k < NIN; k++) {
-        x[k] = a.X[(long)NIN * id + k];
-        if (a.qat) x[k] = bf16_round(x[k]);
-        c[C_X + k] = x[k];
-    }
-    float h1[NH];
-#pragma unroll
-    for (int j = 0; j < NH; j++) {
-        float z = w[OFF_B1 + j];
-#pragma unroll
-        for (int k = 0; k < NIN; k++) z = z + w[OFF_W1 + j * NIN + k] * x[k];
-        float h = fmaxf(z, 0.0f);
-        if (a.qat) h = bf16_round(h);
-        h1[j] = h;
-        c[C_H1 + j] = h;
-    }
-    float y0 = w[OFF_B3], y1 = w[OFF_B3 + 1];
-    for (int j = 0; j < NH; j++) {
-        float z = w[OFF_B2 + j];
-#pragma unroll
-        for (int k = 0; k < NH; k++) z = z + w[OFF_W2 + j * NH + k] * h1[k];
-        float h = fmaxf(z, 0.0f);
-        if (a.qat) h = bf16_round(h);
-        c[C_H2 + j] = h;
-        y0 = y0 + w[OFF_W3 + j] * h;
-        y1 = y1 + w[OFF_W3 + NH + j] * h;
-    }
-    const float t0 = a.T[2 * id];
-    const float e0 = y0 - t0, e1 = y1 - a.T[2 * id + 1];
+
+    // the rows of the two factors of this lane's parameter (rb < 0: factor 1)
+    const int p = tid;
+    int ra = R_L, rb = -1;
+    if (p < OFF_B1) { ra = R_DZ1 + p / NIN; rb = R_X + p % NIN; }
+    else if (p < OFF_W2) { ra = R_DZ1 + (p - OFF_B1); }
+    else if (p < OFF_B2) { ra = R_DZ2 + (p - OFF_W2) / NH; rb = R_H1 + (p - OFF_W2) % NH; }
+    else if (p < OFF_W3) { ra = R_DZ2 + (p - OFF_B2); }
+    else if (p < OFF_B3) { ra = R_DY + (p - OFF_W3) / NH; rb = R_H2 + (p - OFF_W3) % NH; }
+    else if (p < NPARAM) { ra = R_DY + (p - OFF_B3); }
+    float acc = 0.0f;
+
     const float invB = 1.0f / (float)a.B;
-    // q = z e^{t0} = log(W/E): the guess W0 = E e^q misses W by q times the
-    // error of y0, so the hot states (large q) are weighted up
-    float wq = 1.0f;
-    if (a.q_ref > 0.0f) {
-        const float sz = a.X[(long)NIN * id + 2];
-        const float r = sz * sz * expf(t0) / a.q_ref;
-        wq = 1.0f + r * r;
+    for (int c0 = s0; c0 < s1; c0 += TS) {
+        const bool in = c0 + ls < s1;
+        float x[NIN] = {xn.x, xn.y, xn.z, xn.w};
+        const float sz = x[2], t0 = tn.x, t1 = tn.y;
+        if (c0 + TS < s1) gather(c0 + TS + ls);
+#pragma unroll
+        for (int k = 0; k < NIN; k++)
+            if (a.qat) x[k] = bf16_round(x[k]);
+        float h1[4], h2[4], d2[4], dh1[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const float4 w = *reinterpret_cast<const float4 *>(w1 + (4 * q + i) * NIN);
+            float z = b1[4 * q + i];
+            z = z + w.x * x[0];
+            z = z + w.y * x[1];
+            z = z + w.z * x[2];
+            z = z + w.w * x[3];
+            const float h = fmaxf(z, 0.0f);
+            h1[i] = a.qat ? bf16_round(h) : h;
+            h2[i] = b2[4 * q + i];
+            dh1[i] = 0.0f;
+        }
+        each_unit([&](auto k) {
+            constexpr int K = decltype(k)::value;
+            const float h = quad_bcast<K / 4>(h1[K % 4]);
+#pragma unroll
+            for (int i = 0; i < 4; i++) h2[i] = h2[i] + w2[(4 * q + i) * W2ROW + K] * h;
+        });
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const float h = fmaxf(h2[i], 0.0f);
+            h2[i] = a.qat ? bf16_round(h) : h;
+        }
+        float y0 = b3[0], y1 = b3[1];
+        each_unit([&](auto k) {
+            constexpr int K = decltype(k)::value;
+            const float h = quad_bcast<K / 4>(h2[K % 4]);
+            y0 = y0 + w3[K] * h;
+            y1 = y1 + w3[NH + K] * h;
+        });
+        const float e0 = y0 - t0, e1 = y1 - t1;
+        // q = z e^{t0} = log(W/E): the guess W0 = E e^q misses W by q times the
+        // error of y0, so the hot states (large q) are weighted up
+        float wq = 1.0f;
+        if (a.q_ref > 0.0f) {
+            const float r = sz * sz * expf(t0) / a.q_ref;
+            wq = 1.0f + r * r;
+        }
+        const float dy0 = 2.0f * wq * e0 * invB, dy1 = 2.0f * a.w1 * e1 * invB;
+        const float loss = (wq * e0 * e0 + a.w1 * e1 * e1) * invB;
+        // dz2 = (W3^T dy) * [z2 > 0]   (h2 > 0 <=> z2 > 0)
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            d2[i] = h2[i] > 0.0f ? (w3[4 * q + i] * dy0 + w3[NH + 4 * q + i] * dy1) : 0.0f;
+        each_unit([&](auto k) {
+            constexpr int K = decltype(k)::value;
+            const float d = quad_bcast<K / 4>(d2[K % 4]);
+            const float4 w = *reinterpret_cast<const float4 *>(w2 + K * W2ROW + 4 * q);
+            dh1[0] = dh1[0] + w.x * d;
+            dh1[1] = dh1[1] + w.y * d;
+            dh1[2] = dh1[2] + w.z * d;
+            dh1[3] = dh1[3] + w.w * d;
+        });
+        // samples past the slice add +0 to the sums, which changes no bit of
+        // them (a sum that starts at +0 never becomes -0)
+        float *o = act + ls;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            o[(R_H1 + 4 * q + i) * TROW] = in ? h1[i] : 0.0f;
+            o[(R_H2 + 4 * q + i) * TROW] = in ? h2[i] : 0.0f;
+            o[(R_DZ2 + 4 * q + i) * TROW] = in ? d2[i] : 0.0f;
+            o[(R_DZ1 + 4 * q + i) * TROW] = in && h1[i] > 0.0f ? dh1[i] : 0.0f;
+        }
+        o[(R_X + q) * TROW] = in ? (q == 0 ? x[0] : q == 1 ? x[1] : q == 2 ? x[2] : x[3]) : 0.0f;
+        if (q < 3) o[(R_DY + q) * TROW] = in ? (q == 0 ? dy0 : q == 1 ? dy1 : loss) : 0.0f;
+        static_assert(R_L == R_DY + 2, "dy and the loss are written as three rows");
+        __syncthreads();
+        if (p <= NPARAM) {
+            const float4 *A = reinterpret_cast<const float4 *>(act + ra * TROW);
+            const int n4 = (min(s1 - c0, TS) + 3) / 4;
+            if (rb >= 0) {
+                const float4 *Bv = reinterpret_cast<const float4 *>(act + rb * TROW);
+#pragma unroll 4
+                for (int s = 0; s < n4; s++) {
+                    const float4 u = A[s], v = Bv[s];
+                    acc = acc + u.x * v.x;
+                    acc = acc + u.y * v.y;
+                    acc = acc + u.z * v.z;
+                    acc = acc + u.w * v.w;
+                }
+            } else {
+#pragma unroll 4
+                for (int s = 0; s < n4; s++) {
+                    const float4 u = A[s];
+                    acc = acc + u.x;
+                    acc = acc + u.y;
+                    acc = acc + u.z;
+                    acc = acc + u.w;
+                }
+            }
+        }
+        __syncthreads();
     }
-    const float dy0 = 2.0f * wq * e0 * invB, dy1 = 2.0f * a.w1 * e1 * invB;
-    c[C_DY] = dy0;
-    c[C_DY + 1] = dy1;
-    c[C_L] = (wq * e0 * e0 + a.w1 * e1 * e1) * invB;
-    // dz2 = (W3^T dy) * [z2 > 0]   (h2 > 0 <=> z2 > 0)
-    float dh1[NH];
-#pragma unroll
-    for (int k = 0; k < NH; k++) dh1[k] = 0.0f;
-    for (int j = 0; j < NH; j++) {
-        const float h = c[C_H2 + j];
-        const float d = h > 0.0f ? (w[OFF_W3 + j] * dy0 + w[OFF_W3 + NH + j] * dy1) : 0.0f;
-        c[C_DZ2 + j] = d;
-#pragma unroll
-        for (int k = 0; k < NH; k++) dh1[k] = dh1[k] + w[OFF_W2 + j * NH + k] * d;
-    }
-#pragma unroll
-    for (int k = 0; k < NH; k++) c[C_DZ1 + k] = h1[k] > 0.0f ? dh1[k] : 0.0f;
+    if (p <= NPARAM) a.out->part[blockIdx.x][p] = acc;
 }
 
-// Partial gradient sums: thread = parameter (+1 for the loss), blockIdx.y =
-// slice of the batch.  part[slice][NPARAM + 1].
-__global__ void __launch_bounds__(256) k_train_grad_partial(const float *__restrict__ cache, int B, int nsplit,
-                                                            float *__restrict__ part)
+// The last step's update, or (grad != NULL) the gradient itself.
+__global__ void __launch_bounds__(512) k_train_end(AdamArgs a, const TrainState *in, TrainState *out, float *grad)
 {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
+    const int p = threadIdx.x;
     if (p > NPARAM) return;
-    const int per = (B + nsplit - 1) / nsplit;
-    const int s0 = blockIdx.y * per, s1 = min(B, s0 + per);
-    int oa, ob;  // cache offsets of the two factors (ob < 0: factor 1)
-    if (p < OFF_B1) { oa = C_DZ1 + p / NIN; ob = C_X + p % NIN; }
-    else if (p < OFF_W2) { oa = C_DZ1 + (p - OFF_B1); ob = -1; }
-    else if (p < OFF_B2) { oa = C_DZ2 + (p - OFF_W2) / NH; ob = C_H1 + (p - OFF_W2) % NH; }
-    else if (p < OFF_W3) { oa = C_DZ2 + (p - OFF_B2); ob = -1; }
-    else if (p < OFF_B3) { oa = C_DY + (p - OFF_W3) / NH; ob = C_H2 + (p - OFF_W3) % NH; }
-    else if (p < NPARAM) { oa = C_DY + (p - OFF_B3); ob = -1; }
-    else { oa = C_L; ob = -1; }
-    float acc = 0.0f;
-    if (ob >= 0) {
-        for (int s = s0; s < s1; s++) acc = acc + cache[(long)s * C_STRIDE + oa] * cache[(long)s * C_STRIDE + ob];
+    if (grad) {
+        float g = 0.0f;
+        for (int s = 0; s < a.nsplit; s++) g = g + in->part[s][p];
+        grad[p] = g;
     } else {
-        for (int s = s0; s < s1; s++) acc = acc + cache[(long)s * C_STRIDE + oa];
+        due_param(a, in, out, p, true);
     }
-    part[(long)blockIdx.y * (NPARAM + 1) + p] = acc;
-}
-
-__global__ void k_train_grad_final(const float *__restrict__ part, int nsplit, float *__restrict__ grad)
-{
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p > NPARAM) return;
-    float acc = 0.0f;
-    for (int s = 0; s < nsplit; s++) acc = acc + part[(long)s * (NPARAM + 1) + p];
-    grad[p] = acc;
-}
-
-__global__ void k_adam(float *__restrict__ prm, float *__restrict__ m, float *__restrict__ v,
-                       const float *__restrict__ grad, float lr, float b1, float b2, float eps, float bc1,
-                       float bc2, float *loss_out)
-{
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p == NPARAM && loss_out) *loss_out = grad[NPARAM];
-    if (p >= NPARAM) return;
-    const float g = grad[p];
-    const float mm = b1 * m[p] + (1.0f - b1) * g;
-    const float vv = b2 * v[p] + (1.0f - b2) * g * g;
-    m[p] = mm;
-    v[p] = vv;
-    prm[p] = prm[p] - lr * (mm / bc1) / (__builtin_sqrtf(vv / bc2) + eps);
 }
 
 }  // namespace vrn_c4
@@ -882,7 +1012,6 @@ int grid_for(long work, int block, int cap = 8192)
 
 constexpr int MAX_BATCH = 65536;
 constexpr int MAX_SOLVE_GRID = 4096;
-constexpr int NSPLIT = 64;
 }  // namespace
 
 struct vrn_c2p {
@@ -900,7 +1029,8 @@ struct vrn_c2p {
     bool net_ok = false;      // net matches params
     bool have_params = false, have_prev = false, have_P = false, recorded = false;
     // training / test buffers (allocated on first use)
-    float *cache = nullptr, *part = nullptr, *grad = nullptr, *m = nullptr, *v = nullptr, *tprm = nullptr;
+    TrainState *train[2] = {nullptr, nullptr};
+    float *grad = nullptr;
     float *X = nullptr, *T = nullptr;
     int *idx = nullptr;
     unsigned char *valid = nullptr;
@@ -923,13 +1053,10 @@ int ensure_net(vrn_c2p *h)
 
 int ensure_train(vrn_c2p *h)
 {
-    if (h->cache) return 0;
-    HIPCHK(hipMalloc(&h->cache, sizeof(float) * (size_t)C_STRIDE * MAX_BATCH));
-    HIPCHK(hipMalloc(&h->part, sizeof(float) * (size_t)NSPLIT * (NPARAM + 1)));
+    if (h->grad) return 0;
+    for (int k = 0; k < 2; k++)
+        if (!h->train[k]) HIPCHK(hipMalloc(&h->train[k], sizeof(TrainState)));
     HIPCHK(hipMalloc(&h->grad, sizeof(float) * (NPARAM + 1)));
-    HIPCHK(hipMalloc(&h->m, sizeof(float) * NPARAM));
-    HIPCHK(hipMalloc(&h->v, sizeof(float) * NPARAM));
-    HIPCHK(hipMalloc(&h->tprm, sizeof(float) * NPARAM));
     return 0;
 }
 
@@ -957,32 +1084,8 @@ int ensure_pairs(vrn_c2p *h, long n)
     return 0;
 }
 
-// One forward/backward + gradient reduction over B samples (cache -> grad).
-int grad_pass(vrn_c2p *h, const float *X, const float *T, const int *idx, long n_idx, int B,
-              unsigned long long seed, int step, const float *prm, float w1, float q_ref, int qat)
-{
-    TrainArgs ta;
-    ta.X = X;
-    ta.T = T;
-    ta.idx = idx;
-    ta.n_idx = n_idx;
-    ta.B = B;
-    ta.seed = seed;
-    ta.step = step;
-    ta.prm = prm;
-    ta.cache = h->cache;
-    ta.w1 = w1;
-    ta.q_ref = q_ref;
-    ta.qat = qat;
-    hipLaunchKernelGGL(k_train_fwd_bwd, dim3((B + 255) / 256), dim3(256), 0, h->s, ta);
-    const int nsplit = B < NSPLIT ? B : NSPLIT;
-    hipLaunchKernelGGL(k_train_grad_partial, dim3((NPARAM + 1 + 255) / 256, nsplit), dim3(256), 0, h->s,
-                       (const float *)h->cache, B, nsplit, h->part);
-    hipLaunchKernelGGL(k_train_grad_final, dim3((NPARAM + 1 + 255) / 256), dim3(256), 0, h->s,
-                       (const float *)h->part, nsplit, h->grad);
-    HIPCHK(hipGetLastError());
-    return 0;
-}
+// Slices of a batch of B samples.
+int slices(int B) { return B < NSPLIT ? B : NSPLIT; }
 
 // Seeded He initialisation on the host (SplitMix64 + Box-Muller).
 void he_init(std::vector<float> &w, unsigned long long seed)
@@ -1056,12 +1159,9 @@ int vrn_c2p_destroy(vrn_c2p *h)
     (void)hipFree(h->crow);
     (void)hipFree(h->params);
     (void)hipFree(h->net);
-    (void)hipFree(h->cache);
-    (void)hipFree(h->part);
+    (void)hipFree(h->train[0]);
+    (void)hipFree(h->train[1]);
     (void)hipFree(h->grad);
-    (void)hipFree(h->m);
-    (void)hipFree(h->v);
-    (void)hipFree(h->tprm);
     (void)hipFree(h->X);
     (void)hipFree(h->T);
     (void)hipFree(h->idx);
@@ -1267,8 +1367,21 @@ int vrn_mlp_grad(vrn_c2p *h, int64_t n, const float *X, const float *T, const fl
     if (int rc = ensure_pairs(h, n)) return rc;
     HIPCHK(hipMemcpyAsync(h->X, X, sizeof(float) * NIN * (size_t)n, hipMemcpyHostToDevice, h->s));
     HIPCHK(hipMemcpyAsync(h->T, T, sizeof(float) * 2 * (size_t)n, hipMemcpyHostToDevice, h->s));
-    HIPCHK(hipMemcpyAsync(h->tprm, params, sizeof(float) * NPARAM, hipMemcpyHostToDevice, h->s));
-    if (int rc = grad_pass(h, h->X, h->T, nullptr, n, (int)n, 0, 0, h->tprm, 1.0f, q_ref, qat ? 1 : 0)) return rc;
+    HIPCHK(hipMemcpyAsync(h->train[0]->prm, params, sizeof(float) * NPARAM, hipMemcpyHostToDevice, h->s));
+    TrainArgs ta{};
+    ta.X = h->X;
+    ta.T = h->T;
+    ta.B = (int)n;
+    ta.in = h->train[0];
+    ta.out = h->train[1];
+    ta.adam.nsplit = slices((int)n);
+    ta.w1 = 1.0f;
+    ta.q_ref = q_ref;
+    ta.qat = qat ? 1 : 0;
+    hipLaunchKernelGGL(k_train_step, dim3(ta.adam.nsplit), dim3(4 * TS), 0, h->s, ta);
+    hipLaunchKernelGGL(k_train_end, dim3(1), dim3(512), 0, h->s, ta.adam, (const TrainState *)h->train[1], h->train[0],
+                       h->grad);
+    HIPCHK(hipGetLastError());
     std::vector<float> g(NPARAM + 1);
     HIPCHK(hipMemcpyAsync(g.data(), h->grad, sizeof(float) * (NPARAM + 1), hipMemcpyDeviceToHost, h->s));
     HIPCHK(hipStreamSynchronize(h->s));
@@ -1309,24 +1422,52 @@ int vrn_mlp_train(vrn_c2p *h, int64_t n, const double *U, const double *P, const
         he_init(w0, tp->seed);
     }
     h->net_ok = false;
-    HIPCHK(hipMemcpyAsync(h->params, w0.data(), sizeof(float) * NPARAM, hipMemcpyHostToDevice, h->s));
-    HIPCHK(hipMemsetAsync(h->m, 0, sizeof(float) * NPARAM, h->s));
-    HIPCHK(hipMemsetAsync(h->v, 0, sizeof(float) * NPARAM, h->s));
+    HIPCHK(hipMemsetAsync(h->train[0], 0, sizeof(TrainState), h->s));
+    HIPCHK(hipMemcpyAsync(h->train[0]->prm, w0.data(), sizeof(float) * NPARAM, hipMemcpyHostToDevice, h->s));
     float *curve = nullptr;
     HIPCHK(hipMalloc(&curve, sizeof(float) * (size_t)tp->steps));
     double bc1 = 1.0, bc2 = 1.0;
     int rc = 0;
-    for (int s = 0; s < tp->steps && rc == 0; s++) {
+    TrainArgs ta{};
+    ta.X = h->X;
+    ta.T = h->T;
+    ta.idx = h->idx;
+    ta.n_idx = (long)ids.size();
+    ta.B = tp->batch;
+    ta.seed = tp->seed;
+    ta.w1 = tp->w_out1;
+    ta.q_ref = tp->q_ref;
+    ta.qat = tp->qat;
+    AdamArgs &ad = ta.adam;
+    ad.nsplit = slices(tp->batch);
+    ad.b1 = tp->beta1;
+    ad.b2 = tp->beta2;
+    ad.eps = tp->eps;
+    for (int s = 0; s < tp->steps; s++) {
+        ta.step = s;
+        ta.in = h->train[s & 1];
+        ta.out = h->train[(s + 1) & 1];
+        hipLaunchKernelGGL(k_train_step, dim3(ad.nsplit), dim3(4 * TS), 0, h->s, ta);
+        // this step's update, made at the start of the next launch
         const double lr = tp->lr_min + 0.5 * (tp->lr - tp->lr_min) * (1.0 + std::cos(3.141592653589793 * s / tp->steps));
         bc1 *= tp->beta1;
         bc2 *= tp->beta2;
-        rc = grad_pass(h, h->X, h->T, h->idx, (long)ids.size(), tp->batch, tp->seed, s, h->params, tp->w_out1,
-                       tp->q_ref, tp->qat);
-        if (rc) break;
-        hipLaunchKernelGGL(k_adam, dim3((NPARAM + 1 + 255) / 256), dim3(256), 0, h->s, h->params, h->m, h->v,
-                           (const float *)h->grad, (float)lr, tp->beta1, tp->beta2, tp->eps, (float)(1.0 - bc1),
-                           (float)(1.0 - bc2), curve + s);
-        if (hipGetLastError() != hipSuccess) rc = fail(-2, "vrn_mlp_train: launch failed at step %d", s);
+        ad.due = 1;
+        ad.lr = (float)lr;
+        ad.bc1 = (float)(1.0 - bc1);
+        ad.bc2 = (float)(1.0 - bc2);
+        ad.loss_out = curve + s;
+        if (hipGetLastError() != hipSuccess) {
+            rc = fail(-2, "vrn_mlp_train: launch failed at step %d", s);
+            break;
+        }
+    }
+    if (rc == 0) {
+        TrainState *in = h->train[tp->steps & 1], *out = h->train[(tp->steps + 1) & 1];
+        hipLaunchKernelGGL(k_train_end, dim3(1), dim3(512), 0, h->s, ad, (const TrainState *)in, out, (float *)nullptr);
+        if (hipGetLastError() != hipSuccess ||
+            hipMemcpyAsync(h->params, out->prm, sizeof(float) * NPARAM, hipMemcpyDeviceToDevice, h->s) != hipSuccess)
+            rc = fail(-2, "vrn_mlp_train: launch of the last update failed");
     }
     if (rc == 0 && loss_curve)
         rc = hipMemcpyAsync(loss_curve, curve, sizeof(float) * (size_t)tp->steps, hipMemcpyDeviceToHost, h->s) ==
