@@ -55,3 +55,26 @@ def test_training_gradient_of_any_batch(n):
     lr, gr = mlp_ref.loss_grad(params, X, T, qat=False, q_ref=0.01)
     assert abs(loss - lr) <= 1e-4 * lr
     assert np.linalg.norm(g - gr) <= 1e-4 * np.linalg.norm(gr)
+
+
+@pytest.mark.parametrize("scale", [1e-290, 1e-300, 2e-304, 3e-307, 5e-310, 1e-322])
+def test_ppm_fluxes_on_tiny_values(oracle, scale):
+    """The division by six of PPM's interface values where its quotient or
+    the remainder of the correction is subnormal: the oracle's bits."""
+    from helpers import from_oracle3, to_oracle3
+    from verona_amd import DeviceGrid
+    progress(f"ppm on tiny values {scale}")
+    P = state3(20, 12, 9, seed=41)
+    rng = np.random.default_rng(41)
+    P[2:] = scale * rng.standard_normal(P[2:].shape)
+    P[3][rng.random(P[3].shape) < 0.3] = 0.0
+    Po = to_oracle3(P)
+    sl = (slice(None), slice(2, -3), slice(2, -3), slice(2, -3))
+    with DeviceGrid(3, 20, 12, 9, G) as dev:
+        dev.upload("P", P)
+        for dim, slot in enumerate(["Fx", "Fy", "Fz"]):
+            dev.upload(slot, np.zeros_like(P))
+            dev.fluxes(dim, 1e-7, "ppm", "hll")
+            a = dev.download(slot)[sl]
+            b = from_oracle3(oracle.fluxes3(Po, G, 1e-7, dim, "ppm", "hll"))[sl]
+            assert np.array_equal(a, b)

@@ -298,96 +298,99 @@ template <class T> __device__ __forceinline__ void minmod(T qm1, T q, T qp1, T &
     hi = q + dU;
 }
 
-// x / 6.  Fast FP64 form: x (1/6) plus one remainder correction (Markstein:
-// with 1/6 rounded to nearest and a first quotient within an ulp, the
-// corrected quotient is the correctly rounded x / 6 away from the subnormal
-// range); otherwise the IEEE division.
+// x / 6 in FP64: x (1/6) plus one remainder correction (Markstein: with 1/6
+// rounded to nearest and a first quotient within an ulp, the corrected
+// quotient is the correctly rounded x / 6).  Where the remainder is not exact
+// (0 < |x| < 2^-1010) the exact form divides; v_div_fixup gives +-0, +-inf and
+// NaN as the division does.  5 instructions for the division's 11 (FP32: the
+// IEEE division).
 template <class T> __device__ __forceinline__ T div6(T x)
 {
-#if defined(VRN_FAST)
     if constexpr (std::is_same<T, double>::value) {
         constexpr double c = 1.0 / 6.0;
-        const double q = x * c;
-        return __builtin_fma(__builtin_fma(-q, 6.0, x), c, q);
-    }
+        double q = x * c;
+        q = __builtin_fma(__builtin_fma(-q, 6.0, x), c, q);
+#if defined(VRN_FAST)
+        return q;
+#elif defined(__HIP_DEVICE_COMPILE__)
+        q = __builtin_amdgcn_div_fixup(q, 6.0, x);
+        if (dabs(x) < 0x1p-1000)
+            if (x != 0.0) q = x / 6.0;
+        return q;
 #endif
+    }
     return x / T(6);
 }
 
-// fluxlimiter.jl:74-180  PPM (AthenaPK form)
-template <class T>
-__device__ __forceinline__ void ppm(T q_im2, T q_im1, T q_i, T q_ip1, T q_ip2, T &lo, T &hi)
+// fluxlimiter.jl:74-180  PPM (AthenaPK form), in two parts.
+// The limited interface value between q0 and q1 from their neighbours qm and
+// qp: dph of the cell right of the interface and dph_ip1 of the cell left of
+// it are this same value, bit for bit, so a sweep may form it once for both.
+template <class T> __device__ __forceinline__ T ppm_iface(T qm, T q0, T q1, T qp)
 {
     const T C2 = T(1.25);
-    T qa = q_i - q_im1;
-    T qb = q_ip1 - q_i;
-    T dd_im1 = T(0.5) * qa + T(0.5) * (q_im1 - q_im2);
-    T dd = T(0.5) * qb + T(0.5) * qa;
-    T dd_ip1 = T(0.5) * (q_ip2 - q_ip1) + T(0.5) * qb;
-    T dph = T(0.5) * (q_im1 + q_i) + div6(dd_im1 - dd);
-    T dph_ip1 = T(0.5) * (q_i + q_ip1) + div6(dd - dd_ip1);
-    T d2qc_im1 = q_im2 + q_i - T(2) * q_im1;
-    T d2qc = q_im1 + q_ip1 - T(2) * q_i;
-    T d2qc_ip1 = q_i + q_ip2 - T(2) * q_ip1;
+    const T d = q1 - q0;
+    const T d0 = T(0.5) * d + T(0.5) * (q0 - qm);
+    const T d1 = T(0.5) * (qp - q1) + T(0.5) * d;
+    T f = T(0.5) * (q0 + q1) + div6(d0 - d1);
+    // only an overshoot is limited; waves without one skip it
+    if ((f - q0) * (q1 - f) < T(0)) {
+        const T qa = T(3) * (q0 + q1 - T(2) * f);
+        const T qb = qm + q1 - T(2) * q0;
+        const T qc = q0 + qp - T(2) * q1;
+        T qd = T(0);
+        // sign(qa) * min(...) with equal signs: the min is +0 exactly when qa
+        // is +-0, so the product is copysign(min, qa)
+        if (same_sign3(qa, qb, qc))
+            qd = __builtin_copysign(nn_min(C2 * dabs(qb), nn_min(C2 * dabs(qc), dabs(qa))), qa);
+        f = T(0.5) * (q0 + q1) - div6(qd);
+    }
+    return f;
+}
 
-    T qa_tmp = dph - q_im1;
-    T qb_tmp = q_i - dph;
-    qa = T(3) * (q_im1 + q_i - T(2) * dph);
-    qb = d2qc_im1;
-    T qc = d2qc;
-    T qd = T(0);
-    // sign(qa) * min(...) with equal signs: the min is +0 exactly when qa is
-    // +-0, so the product is copysign(min, qa)
-    if (same_sign3(qa, qb, qc))
-        qd = __builtin_copysign(nn_min(C2 * dabs(qb), nn_min(C2 * dabs(qc), dabs(qa))), qa);
-    T dph_tmp = T(0.5) * (q_im1 + q_i) - div6(qd);
-    if (qa_tmp * qb_tmp < T(0)) dph = dph_tmp;
-
-    qa_tmp = dph_ip1 - q_i;
-    qb_tmp = q_ip1 - dph_ip1;
-    qa = T(3) * (q_i + q_ip1 - T(2) * dph_ip1);
-    qb = d2qc;
-    qc = d2qc_ip1;
-    qd = T(0);
-    if (same_sign3(qa, qb, qc))
-        qd = __builtin_copysign(nn_min(C2 * dabs(qb), nn_min(C2 * dabs(qc), dabs(qa))), qa);
-    T dphip1_tmp = T(0.5) * (q_i + q_ip1) - div6(qd);
-    if (qa_tmp * qb_tmp < T(0)) dph_ip1 = dphip1_tmp;
-
-    T d2qf = T(6) * (dph + dph_ip1 - T(2) * q_i);
+// Face values of cell q_i from its limited interface values dph (left) and
+// dph_ip1 (right).
+template <class T>
+__device__ __forceinline__ void ppm_cell(T q_im2, T q_im1, T q_i, T q_ip1, T q_ip2, T dph, T dph_ip1, T &lo, T &hi)
+{
+    const T C2 = T(1.25);
     T qr_i = dph, ql_ip1 = dph_ip1;
-    T dqf_minus = q_i - qr_i;
-    T dqf_plus = ql_ip1 - q_i;
-    qa_tmp = dqf_minus * dqf_plus;
-    qb_tmp = (q_ip1 - q_i) * (q_i - q_im1);
-    qa = d2qc_im1;
-    qb = d2qc;
-    qc = d2qc_ip1;
-    qd = d2qf;
-    T qe = T(0);
-    if (same_sign4(qa, qb, qc, qd))
-        qe = __builtin_copysign(nn_min(nn_min(C2 * dabs(qa), C2 * dabs(qb)), nn_min(C2 * dabs(qc), dabs(qd))), qd);
-    // a NaN among the five inputs makes qd = d2qf NaN, so the test below is
-    // false whatever the maximum: Julia's NaN-propagating max is not needed
-    qa = nn_max(dabs(q_im1), dabs(q_im2));
-    qb = nn_max(nn_max(dabs(q_i), dabs(q_ip1)), dabs(q_ip2));
-    T rho = T(0);
-    if (dabs(qd) > T(1.0e-12) * nn_max(qa, qb)) rho = qe / qd;
-    T tmp_m = q_i - rho * dqf_minus;
-    T tmp_p = q_i + rho * dqf_plus;
-    T tmp2_m = q_i - T(2) * dqf_plus;
-    T tmp2_p = q_i + T(2) * dqf_minus;
-    if (qa_tmp <= T(0) || qb_tmp <= T(0)) {
+    const T dqf_minus = q_i - qr_i;
+    const T dqf_plus = ql_ip1 - q_i;
+    // extrema and monotone cells each have a part of their own: most waves
+    // are all monotone and skip the first (rho needs four second differences
+    // and a division)
+    if (dqf_minus * dqf_plus <= T(0) || (q_ip1 - q_i) * (q_i - q_im1) <= T(0)) {
+        const T qa = q_im2 + q_i - T(2) * q_im1;
+        const T qb = q_im1 + q_ip1 - T(2) * q_i;
+        const T qc = q_i + q_ip2 - T(2) * q_ip1;
+        const T qd = T(6) * (dph + dph_ip1 - T(2) * q_i);
+        T qe = T(0);
+        if (same_sign4(qa, qb, qc, qd))
+            qe = __builtin_copysign(nn_min(nn_min(C2 * dabs(qa), C2 * dabs(qb)), nn_min(C2 * dabs(qc), dabs(qd))), qd);
+        // a NaN among the five inputs makes qd NaN, so the test below is false
+        // whatever the maximum: Julia's NaN-propagating max is not needed
+        const T big = nn_max(nn_max(dabs(q_im1), dabs(q_im2)),
+                             nn_max(nn_max(dabs(q_i), dabs(q_ip1)), dabs(q_ip2)));
+        T rho = T(0);
+        if (dabs(qd) > T(1.0e-12) * big) rho = qe / qd;
         if (rho <= T(1) - T(1.0e-12)) {
-            qr_i = tmp_m;
-            ql_ip1 = tmp_p;
+            qr_i = q_i - rho * dqf_minus;
+            ql_ip1 = q_i + rho * dqf_plus;
         }
     } else {
-        if (dabs(dqf_minus) >= T(2) * dabs(dqf_plus)) qr_i = tmp2_m;
-        if (dabs(dqf_plus) >= T(2) * dabs(dqf_minus)) ql_ip1 = tmp2_p;
+        if (dabs(dqf_minus) >= T(2) * dabs(dqf_plus)) qr_i = q_i - T(2) * dqf_plus;
+        if (dabs(dqf_plus) >= T(2) * dabs(dqf_minus)) ql_ip1 = q_i + T(2) * dqf_minus;
     }
     lo = qr_i;
     hi = ql_ip1;
+}
+
+template <class T>
+__device__ __forceinline__ void ppm(T q_im2, T q_im1, T q_i, T q_ip1, T q_ip2, T &lo, T &hi)
+{
+    ppm_cell(q_im2, q_im1, q_i, q_ip1, q_ip2, ppm_iface(q_im2, q_im1, q_i, q_ip1), ppm_iface(q_im1, q_i, q_ip1, q_ip2),
+             lo, hi);
 }
 
 template <int REC, class T>

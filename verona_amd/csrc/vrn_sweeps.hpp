@@ -396,7 +396,11 @@ __global__ __launch_bounds__(256, VRN_MARCH_MIN_WAVES) void k_march(SweepArgs a)
     // WENO-Z: the curvature term of each cell (wz_curv) is computed once and
     // carried: cell c needs the terms of cells c-1, c and c+1, and the term of
     // cell x lives in slot x & 1 of a two-slot ring [slot][var][lane].
+    // PPM: the limited interface value right of a cell is the next cell's left
+    // one (ppm_iface): formed once, carried in registers along the march and,
+    // in the x part, taken from the left lane.
     constexpr bool CARRY = REC == REC_WENOZ;
+    constexpr bool PPMC = REC == REC_PPM;
     __shared__ R curv[CARRY ? 2 * NV * WS : 1];
     const Geo G = a.geo;
     const int tid = threadIdx.x;
@@ -431,6 +435,7 @@ __global__ __launch_bounds__(256, VRN_MARCH_MIN_WAVES) void k_march(SweepArgs a)
     R *kl = curv + tid;  // curvature term of cell x, variable v at kl[((x & 1) * NV + v) * WS]
 
     // ring: cell m lives in slot (m - (m0 - 3)) mod 5
+    R pif[NV];  // PPM: interface value left of cell c
     double nx[NV];
 #pragma unroll
     for (int v = 0; v < NV; v++) {
@@ -445,6 +450,9 @@ __global__ __launch_bounds__(256, VRN_MARCH_MIN_WAVES) void k_march(SweepArgs a)
             kl[(((m0 - 1) & 1) * NV + v) * WS] =
                 wz_curv(wl[(1 * NV + v) * WSR], wl[(2 * NV + v) * WSR], wl[(3 * NV + v) * WSR]);
         }
+        if constexpr (PPMC)
+            pif[v] = ppm_iface(wl[(0 * NV + v) * WSR], wl[(1 * NV + v) * WSR], wl[(2 * NV + v) * WSR],
+                               wl[(3 * NV + v) * WSR]);
     }
     const int wv = tid >> 6;
     // XY: the edge face that is this lane's left face (-1: solved in the
@@ -499,6 +507,12 @@ __global__ __launch_bounds__(256, VRN_MARCH_MIN_WAVES) void k_march(SweepArgs a)
                 const R km = *kp, k0 = kl[((c & 1) * NV + v) * WS], kn = wz_curv(q2, q3, q4);
                 *kp = kn;
                 wenoz_k(wl[(s0 * NV + v) * WSR], wl[(s1 * NV + v) * WSR], q2, q3, q4, km, k0, kn, lo[v], up[v]);
+            } else if constexpr (PPMC) {
+                const R q1 = wl[(s1 * NV + v) * WSR], q2 = wl[(s2 * NV + v) * WSR];
+                const R q3 = wl[(s3 * NV + v) * WSR], q4 = wl[(s4 * NV + v) * WSR];
+                const R fr = ppm_iface(q1, q2, q3, q4);
+                ppm_cell(wl[(s0 * NV + v) * WSR], q1, q2, q3, q4, pif[v], fr, lo[v], up[v]);
+                pif[v] = fr;
             } else {
                 recon<REC>(wl[(s0 * NV + v) * WSR], wl[(s1 * NV + v) * WSR], wl[(s2 * NV + v) * WSR],
                            wl[(s3 * NV + v) * WSR], wl[(s4 * NV + v) * WSR], lo[v], up[v]);
@@ -539,7 +553,13 @@ __global__ __launch_bounds__(256, VRN_MARCH_MIN_WAVES) void k_march(SweepArgs a)
 #pragma unroll
                     for (int v = 0; v < NV; v++) {
                         const R *rw = wl + (s1 * NV + v) * WSR;
-                        recon<REC>(rw[-2], rw[-1], rw[0], rw[1], rw[2], lox[v], upx[v]);
+                        if constexpr (PPMC) {
+                            // lane 0's left value is wrong; its faces are edge faces
+                            const R fr = ppm_iface(rw[-1], rw[0], rw[1], rw[2]);
+                            ppm_cell(rw[-2], rw[-1], rw[0], rw[1], rw[2], shift_up1(fr, fr), fr, lox[v], upx[v]);
+                        } else {
+                            recon<REC>(rw[-2], rw[-1], rw[0], rw[1], rw[2], lox[v], upx[v]);
+                        }
                     }
                     lox[0] = floor_max(fl, lox[0]);
                     lox[1] = floor_max(fl, lox[1]);
