@@ -230,7 +230,10 @@ int vrn_tubes_set_method(vrn_tubes *tb, int rec, int riemann, int n_iter, double
 int vrn_tubes_set_precision(vrn_tubes *tb, int precision);
 /* Advance all tubes by nsteps midpoint-RK2 steps with `grid` persistent
  * workgroups of `block` threads (multiple of 64); use_graph replays a
- * captured hipGraph.  *ms receives the device time.  Blocks. */
+ * captured hipGraph.  Batches of tubes too few or too uneven to fill the GPU
+ * that way are split into ranges of tubes with overlapping halos instead
+ * (the same bits), in launches whose shape the library chooses.
+ * *ms receives the device time.  Blocks. */
 int vrn_tubes_run(vrn_tubes *tb, int nsteps, int block, int grid, int use_graph, double *ms);
 /* restore = 0 saves (P, U), restore = 1 puts them back (used by the autotuner). */
 int vrn_tubes_checkpoint(vrn_tubes *tb, int restore);

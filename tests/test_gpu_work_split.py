@@ -78,3 +78,31 @@ def test_ppm_fluxes_on_tiny_values(oracle, scale):
             a = dev.download(slot)[sl]
             b = from_oracle3(oracle.fluxes3(Po, G, 1e-7, dim, "ppm", "hll"))[sl]
             assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("rec,riemann", [("ppm", "hllc"), ("wenoz", "hll"), ("minmod", "hllc")])
+@pytest.mark.parametrize("lengths", [[8], [62], [63, 9], [248], [249], [250, 8, 247], [300, 17, 1001], [2000]])
+def test_tubes_split_over_workgroups(oracle, rec, riemann, lengths):
+    """Tubes around the cells a wave (62) and a workgroup (248) hold, in
+    ranges with halos, for step counts that leave a short last launch: the
+    oracle's bits."""
+    from test_gpu_tubes import _oracle_tubes
+    from verona_amd.tubes import Tubes
+    progress(f"split tubes {lengths} {rec} {riemann}")
+    rng = np.random.default_rng(3)
+    lengths = np.array(lengths)
+    n = int(lengths.sum())
+    x = np.concatenate([(np.arange(L) + 0.5) / L for L in lengths])
+    rho = np.where(x < 0.4, 1.0, 0.3) * (1 + 0.1 * rng.standard_normal(n))
+    u = np.where(x < 0.6, 2.0, 0.5) * (1 + 0.1 * rng.standard_normal(n))
+    ux = 0.3 * np.sin(9 * x) + 0.02 * rng.standard_normal(n)
+    dx = 1.0 / lengths
+    dt = 0.3 * dx
+    with Tubes(lengths) as tb:
+        tb.upload(rho, u, ux, dt, dx)
+        tb.set_method(rec, riemann, 50, 1e-10)
+        for k in (1, 18, 4):
+            tb.run(k)
+        got = np.stack(tb.download())
+    want = _oracle_tubes(oracle, lengths, rho, u, ux, dt, dx, 5.0 / 3.0, rec, riemann, 23)
+    assert np.array_equal(got, want, equal_nan=True)

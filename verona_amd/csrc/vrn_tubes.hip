@@ -34,6 +34,7 @@
 #include <vector>
 
 // fast FP64 form of the tube kernels (vrn_tubes_fast.hip)
+void vrn_fast_launch_tubes_split(hipStream_t s, const vrn::TubeArgs &a, int rec, int riem, int block, int nseg);
 void vrn_fast_launch_tubes(hipStream_t s, const vrn::TubeArgs &a, int rec, int riem, int block, int grid);
 
 using namespace vrn;
@@ -77,8 +78,62 @@ struct vrn_tubes {
     int g_block = 0, g_grid = 0, g_steps = 0, g_rec = -1, g_riem = -1, g_prec = -1;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     float last_ms = 0.f;
+    // k_tubes_split: steps a launch (0: whole tubes by k_tubes) and ranges
+    int split_k = 0, nseg = 0;
+    TubeSeg *seg = nullptr;
     double *Psave[3] = {nullptr, nullptr, nullptr}, *Usave[3] = {nullptr, nullptr, nullptr};
 };
+
+namespace {
+
+constexpr int SPLIT_BLOCK = 256;
+constexpr int SPLIT_CELLS = 62 * (SPLIT_BLOCK / 64);
+
+// Ranges for k_tubes_split at k steps a launch (tubes that fit a workgroup
+// whole need no halo); the cells they hold in all, halos included.
+long split_ranges(const int64_t *lengths, const std::vector<int> &order, int k, std::vector<TubeSeg> *out)
+{
+    const int halo = 2 * TUBE_REACH * k, useful = SPLIT_CELLS - 2 * halo;
+    long cells = 0;
+    for (int t : order) {
+        const long N = lengths[t];
+        const long n = N <= SPLIT_CELLS ? 1 : (N + useful - 1) / useful;
+        cells += N + (n - 1) * 2 * halo;
+        if (out)
+            for (long j = 0; j < n; j++) out->push_back({t, (int)(N * j / n), (int)(N * (j + 1) / n)});
+    }
+    return cells;
+}
+
+// How a batch is run: 0 for whole tubes by persistent workgroups (k_tubes),
+// else the steps a launch of k_tubes_split and its ranges.  Persistent
+// workgroups take about 8 us a stage for each 256 cells of the longest tube,
+// and 3.9e-5 us a cell when the chip is full; ranges take at least 6 us a
+// stage, 4.4e-5 us a cell (halos included) and 3 us a launch.  So split
+// ranges win while tubes are too few or too uneven to fill the chip, and
+// persistent workgroups when it is full.  Measured, exact PPM + HLLC, 32
+// steps, persistent / split: 8 tubes of 1000 to 3000 cells 3.29 / 0.41 ms;
+// 256 of 4000 8.8 / 3.4; 1024 of 256 to 8192 17.2 / 13.3; 2000 of 100 to 700
+// (HLL) 3.15 / 3.40; 1280 of 500 2.22 / 2.87; 4096 of 256 to 8192 43.9 / 50.4.
+int split_plan(int ntubes, const int64_t *lengths, const std::vector<int> &order, std::vector<TubeSeg> &seg)
+{
+    long total = 0;
+    for (int t = 0; t < ntubes; t++) total += lengths[t];
+    const double whole = std::max(8.0 * (double)((lengths[order[0]] + 255) / 256), 3.9e-5 * (double)total);
+    int best = 0;
+    double least = whole;
+    for (int k = 1; k <= 16; k *= 2) {
+        const double stage = std::max(6.0, 4.4e-5 * (double)split_ranges(lengths, order, k, nullptr)) + 1.5 / k;
+        if (stage < least) {
+            least = stage;
+            best = k;
+        }
+    }
+    if (best) split_ranges(lengths, order, best, &seg);
+    return best;
+}
+
+}  // namespace
 
 extern "C" {
 
@@ -102,16 +157,31 @@ int vrn_tubes_create(int ntubes, const int64_t *lengths, double gamma, vrn_tubes
     std::vector<int> order(ntubes);
     std::iota(order.begin(), order.end(), 0);
     std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return lengths[a] > lengths[b]; });
-    size_t nd = (size_t)total * 21;  // P, Ph, U, Uh, P0, Psave, Usave x 3 variables
+    std::vector<TubeSeg> seg;
+    c->split_k = split_plan(ntubes, lengths, order, seg);
+    c->nseg = (int)seg.size();
+    // one allocation for the state (P, Ph, U, Uh, P0, Psave, Usave x 3
+    // variables) and the tables, the constant ones of which (off, order, seg)
+    // are copied together
+    const size_t nd = (size_t)total * 21, nt = (size_t)ntubes;
+    const size_t b_off = sizeof(long) * (nt + 1), b_seg = sizeof(TubeSeg) * seg.size(), b_ord = sizeof(int) * nt;
+    std::vector<char> tab(b_off + b_seg + b_ord);
+    std::memcpy(tab.data(), off.data(), b_off);
+    if (b_seg) std::memcpy(tab.data() + b_off, seg.data(), b_seg);
+    std::memcpy(tab.data() + b_off + b_seg, order.data(), b_ord);
     hipError_t e = hipStreamCreate(&c->s);
-    if (e == hipSuccess) e = hipMalloc(&c->buf, nd * sizeof(double));
-    if (e == hipSuccess) e = hipMalloc(&c->off, sizeof(long) * (ntubes + 1));
-    if (e == hipSuccess) e = hipMalloc(&c->order, sizeof(int) * ntubes);
-    if (e == hipSuccess) e = hipMalloc(&c->dt, sizeof(double) * ntubes);
-    if (e == hipSuccess) e = hipMalloc(&c->dx, sizeof(double) * ntubes);
-    if (e == hipSuccess) e = hipMalloc(&c->queue, sizeof(unsigned int));
-    if (e == hipSuccess) e = hipMemcpy(c->off, off.data(), sizeof(long) * (ntubes + 1), hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(c->order, order.data(), sizeof(int) * ntubes, hipMemcpyHostToDevice);
+    if (e == hipSuccess)
+        e = hipMalloc(&c->buf, sizeof(double) * (nd + 2 * nt) + tab.size() + sizeof(unsigned int));
+    if (e == hipSuccess) {
+        c->dt = c->buf + nd;
+        c->dx = c->dt + nt;
+        char *t = reinterpret_cast<char *>(c->dx + nt);
+        c->off = reinterpret_cast<long *>(t);
+        c->seg = reinterpret_cast<TubeSeg *>(t + b_off);
+        c->order = reinterpret_cast<int *>(t + b_off + b_seg);
+        c->queue = reinterpret_cast<unsigned int *>(t + b_off + b_seg + b_ord);
+        e = hipMemcpy(t, tab.data(), tab.size(), hipMemcpyHostToDevice);
+    }
     if (e == hipSuccess) e = hipEventCreate(&c->ev0);
     if (e == hipSuccess) e = hipEventCreate(&c->ev1);
     if (e != hipSuccess) {
@@ -147,11 +217,6 @@ int vrn_tubes_destroy(vrn_tubes *c)
     if (c->ev0) (void)hipEventDestroy(c->ev0);
     if (c->ev1) (void)hipEventDestroy(c->ev1);
     (void)hipFree(c->buf);
-    (void)hipFree(c->off);
-    (void)hipFree(c->order);
-    (void)hipFree(c->dt);
-    (void)hipFree(c->dx);
-    (void)hipFree(c->queue);
     if (c->s) (void)hipStreamDestroy(c->s);
     delete c;
     return 0;
@@ -221,8 +286,36 @@ static void launch_tubes(vrn_tubes *c, int block, int grid)
         vrn::launch_tubes_kernels(c->s, c->args, c->rec, c->riemann, block, grid);
 }
 
-// Advance every tube by nsteps steps with `grid` persistent workgroups of
-// `block` threads.  use_graph != 0 captures (queue reset + persistent kernel)
+// nsteps steps by k_tubes_split, split_k steps a launch (all of them where
+// every tube lies in one workgroup).  The two state buffers change places at
+// each launch.
+static int run_split(vrn_tubes *c, int nsteps)
+{
+    const int most = c->nseg == c->ntubes ? std::max(nsteps, 1) : c->split_k;
+    for (int done = 0; done < nsteps;) {
+        TubeArgs &a = c->args;
+        a.seg = c->seg;
+        a.ksteps = std::min(most, nsteps - done);
+        for (int v = 0; v < 3; v++) {
+            a.Pn[v] = a.Ph[v];
+            a.Un[v] = a.Uh[v];
+        }
+        if (c->precision == VRN_PREC_FP64_FAST)
+            vrn_fast_launch_tubes_split(c->s, a, c->rec, c->riemann, SPLIT_BLOCK, c->nseg);
+        else
+            vrn::launch_tubes_split(c->s, a, c->rec, c->riemann, SPLIT_BLOCK, c->nseg);
+        TCHK(hipGetLastError());
+        for (int v = 0; v < 3; v++) {
+            std::swap(a.P[v], a.Ph[v]);
+            std::swap(a.U[v], a.Uh[v]);
+        }
+        done += a.ksteps;
+    }
+    return 0;
+}
+
+// Advance every tube by nsteps steps: split over workgroups where split_plan
+// says so, else with `grid` persistent workgroups of `block` threads.  use_graph != 0 captures (queue reset + persistent kernel)
 // into a hipGraph once per (block, grid, nsteps, method, precision) and replays it.
 // *ms (may be NULL) receives the device time of the launch.  Blocks.
 int vrn_tubes_run(vrn_tubes *c, int nsteps, int block, int grid, int use_graph, double *ms)
@@ -231,7 +324,11 @@ int vrn_tubes_run(vrn_tubes *c, int nsteps, int block, int grid, int use_graph, 
     if (nsteps < 0 || block < 64 || block > 1024 || (block & 63) || grid < 1)
         return tfail(VRN_E_ARG, "bad launch shape (block %d, grid %d)", block, grid);
     c->args.nsteps = nsteps;
-    if (use_graph) {
+    if (c->split_k) {
+        TCHK(hipEventRecord(c->ev0, c->s));
+        if (int r = run_split(c, nsteps)) return r;
+        TCHK(hipEventRecord(c->ev1, c->s));
+    } else if (use_graph) {
         bool stale = !c->gexec || c->g_block != block || c->g_grid != grid || c->g_steps != nsteps ||
                      c->g_rec != c->rec || c->g_riem != c->riemann || c->g_prec != c->precision;
         if (stale) {

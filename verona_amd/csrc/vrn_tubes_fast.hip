@@ -14,3 +14,8 @@ void vrn_fast_launch_tubes(hipStream_t s, const vrn::TubeArgs &a, int rec, int r
 {
     vrn_fast::launch_tubes_kernels(s, a, rec, riem, block, grid);
 }
+
+void vrn_fast_launch_tubes_split(hipStream_t s, const vrn::TubeArgs &a, int rec, int riem, int block, int nseg)
+{
+    vrn_fast::launch_tubes_split(s, a, rec, riem, block, nseg);
+}

@@ -110,6 +110,25 @@ __device__ __forceinline__ void rec_range(int N, int &lo, int &hi)
     }
 }
 
+// Values of the lanes left and right (DPP wave shifts; lane 0 / 63 keep their
+// own).
+__device__ __forceinline__ double tube_shift_up(double v)
+{
+    const long long b = __double_as_longlong(v);
+    const int lo = (int)(b & 0xffffffffll), hi = (int)(b >> 32);
+    const int l = __builtin_amdgcn_update_dpp(lo, lo, 0x138, 0xf, 0xf, false);
+    const int h = __builtin_amdgcn_update_dpp(hi, hi, 0x138, 0xf, 0xf, false);
+    return __longlong_as_double(((long long)h << 32) | (unsigned int)l);
+}
+__device__ __forceinline__ double tube_shift_down(double v)
+{
+    const long long b = __double_as_longlong(v);
+    const int lo = (int)(b & 0xffffffffll), hi = (int)(b >> 32);
+    const int l = __builtin_amdgcn_update_dpp(lo, lo, 0x130, 0xf, 0xf, false);
+    const int h = __builtin_amdgcn_update_dpp(hi, hi, 0x130, 0xf, 0xf, false);
+    return __longlong_as_double(((long long)h << 32) | (unsigned int)l);
+}
+
 // One RK stage of one tube by the whole workgroup.  s = 0: Pin = P, out to
 // (Uh, Ph) with coefficient 0.5*dt/dx; s = 1: Pin = Ph, out to (U, P) with dt/dx.
 template <int REC, int RIEM>
@@ -223,6 +242,131 @@ __global__ void k_tubes(vrn::TubeArgs a)
     }
 }
 
+// Cells by which one RK stage's stencil reaches out: the faces of a cell
+// need the reconstructions of its neighbours.
+constexpr int TUBE_REACH = 3;
+
+// Steps of a few tubes, or of very uneven ones, leave most of the chip idle
+// when a workgroup takes a whole tube: a stage of the 1024-cell shock tube
+// took 10 us on one CU, four waves to a SIMD.  Here a workgroup takes a range
+// of a tube for ksteps steps, its state in registers.  The range is
+// extended by 2 TUBE_REACH ksteps cells to each side (less where the tube
+// ends), cells next to a cut end keep their state, and what that spoils is
+// never written: only the range itself is, to the other state buffers, which
+// the next launch reads.  A lane holds one cell.  A wave's 64 lanes overlap
+// the next wave's by two, so that it needs nothing of its neighbours but
+// primitives: lanes 0..63 reconstruct, upper states and fluxes go to the
+// next lanes by DPP, lanes 1..62 update.  One barrier a stage, P through LDS
+// in two alternating copies.  What bounds it then is one wave's chain of
+// divisions and square roots: 1024 cells, exact minmod + HLLC, 3.8 us a stage
+// (20.4 -> 7.6 us a step); in full batches the VALU issue.
+template <int REC, int RIEM>
+__global__ __launch_bounds__(1024) void k_tubes_split(vrn::TubeArgs a)
+{
+    extern __shared__ double lds[];
+    __shared__ double ends[3][5];  // first primitives of cells 0, 1, N-3, N-2, N-1
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int cap = 62 * (blockDim.x >> 6) + 6;
+    const vrn::TubeSeg sg = a.seg[blockIdx.x];
+    const int tb = sg.tube;
+    const long o = a.off[tb];
+    const int N = (int)(a.off[tb + 1] - o);
+    const int halo = 2 * TUBE_REACH * a.ksteps;
+    const int own1 = sg.hi;
+    const int e0 = max(0, sg.lo - halo), e1 = min(N, own1 + halo);
+    const double g = a.g;
+    const double dtdx = a.dt[tb] / a.dx[tb], hdtdx = 0.5 * a.dt[tb] / a.dx[tb];
+    int rlo, rhi;
+    rec_range<REC>(N, rlo, rhi);
+
+    const int c = e0 + 62 * wave + lane - 1;
+    const int li = c - e0 + 3;  // its place in a copy of P
+    const bool cell = lane >= 1 && lane <= 62 && c >= e0 && c < e1;
+    const bool upd = cell && c >= 1 && c < N - 2 && (e0 == 0 || c >= e0 + TUBE_REACH) &&
+                     (e1 == N || c < e1 - TUBE_REACH);
+    const bool rec = c >= rlo && c < rhi;
+    double P[3], U[3];
+#pragma unroll
+    for (int v = 0; v < 3; v++) {
+        P[v] = cell ? a.P[v][o + c] : 1.0;
+        U[v] = cell ? a.U[v][o + c] : 1.0;
+    }
+    // places beyond the range hold a state at rest; nothing of them is kept
+    for (int i = tid; i < 6 * cap; i += blockDim.x) lds[i] = (i / cap) % 3 == 2 ? 0.0 : 1.0;
+    if (tid < 15) {
+        const int v = tid / 5, k = tid % 5;
+        ends[v][k] = a.P0[v][o + (k < 2 ? k : N - 5 + k)];
+    }
+    __syncthreads();
+    if (cell) {
+#pragma unroll
+        for (int v = 0; v < 3; v++) lds[v * cap + li] = P[v];
+    }
+    // waves past the range's end only keep the barriers
+    const bool live = e0 + 62 * wave < e1;
+    int b = 0;
+    for (int st = 0; st < 2 * a.ksteps; st++) {
+        __syncthreads();
+        if (!live) continue;
+        const double *sP = lds + b * 3 * cap;
+        double PLc[3], PRm[3];  // PL[c], PR[c-1]
+        if (rec) {
+#pragma unroll
+            for (int v = 0; v < 3; v++) {
+                const double *q = sP + v * cap + li;
+                double lo, hi;
+                if (REC == REC_MINMOD)
+                    minmod(q[-1], q[0], q[1], lo, hi);
+                else
+                    recon<REC>(q[-2], q[-1], q[0], q[1], q[2], lo, hi);
+                PLc[v] = hi;
+                PRm[v] = lo;
+            }
+        } else {
+            // never reconstructed: the first primitives (lanes off the tube: any)
+            const int k = c < 2 ? max(c, 0) : min(max(c - (N - 5), 2), 4);
+            const int km = c < 3 ? max(c - 1, 0) : min(max(c - 1 - (N - 5), 2), 4);
+#pragma unroll
+            for (int v = 0; v < 3; v++) {
+                PLc[v] = ends[v][k];
+                PRm[v] = ends[v][km];
+            }
+        }
+        double PLm[3], F[3];
+#pragma unroll
+        for (int v = 0; v < 3; v++) PLm[v] = tube_shift_up(PLc[v]);
+        face1<RIEM>(PLm, PRm, g, F);  // face c - 1/2
+        const double coef = (st & 1) ? dtdx : hdtdx;
+        double Uo[3], x[3];
+#pragma unroll
+        for (int v = 0; v < 3; v++) {
+            const double Fr = tube_shift_down(F[v]);
+            Uo[v] = upd ? U[v] - coef * (Fr - F[v]) : U[v];
+            x[v] = P[v];
+        }
+        b ^= 1;
+        if (cell) {
+            c2p1(Uo, x, g, a.n_iter, a.tol);
+#pragma unroll
+            for (int v = 0; v < 3; v++) lds[(b * 3 + v) * cap + li] = x[v];
+        }
+        if (st & 1) {
+#pragma unroll
+            for (int v = 0; v < 3; v++) {
+                P[v] = x[v];
+                U[v] = Uo[v];
+            }
+        }
+    }
+    if (cell && c >= sg.lo && c < own1) {
+#pragma unroll
+        for (int v = 0; v < 3; v++) {
+            a.Pn[v][o + c] = P[v];
+            a.Un[v][o + c] = U[v];
+        }
+    }
+}
+
 #if !defined(VRN_FAST)
 // U = PtoU(P) on every cell (1dim/structs.jl:58-66), Uhalf = U.  Part of the
 // upload, so both arithmetic forms start from the exact-form U.
@@ -262,6 +406,23 @@ inline void launch_tubes_kernels(hipStream_t s, const vrn::TubeArgs &a, int rec,
         else VRN_TL(REC_MINMOD, RIEM_HLLC);
     }
 #undef VRN_TL
+}
+
+// One launch of k_tubes_split over nseg ranges.
+inline void launch_tubes_split(hipStream_t s, const vrn::TubeArgs &a, int rec, int riem, int block, int nseg)
+{
+    const size_t lds = sizeof(double) * 6 * (62 * (block / 64) + 6);
+#define VRN_TS(R_, M_) hipLaunchKernelGGL((k_tubes_split<R_, M_>), dim3(nseg), dim3(block), lds, s, a)
+    if (riem == RIEM_HLL) {
+        if (rec == REC_PPM) VRN_TS(REC_PPM, RIEM_HLL);
+        else if (rec == REC_WENOZ) VRN_TS(REC_WENOZ, RIEM_HLL);
+        else VRN_TS(REC_MINMOD, RIEM_HLL);
+    } else {
+        if (rec == REC_PPM) VRN_TS(REC_PPM, RIEM_HLLC);
+        else if (rec == REC_WENOZ) VRN_TS(REC_WENOZ, RIEM_HLLC);
+        else VRN_TS(REC_MINMOD, RIEM_HLLC);
+    }
+#undef VRN_TS
 }
 
 }  // namespace VRN_NS

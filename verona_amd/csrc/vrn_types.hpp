@@ -76,6 +76,11 @@ struct SweepArgs {
     int xmap_lo, xmap_hi;
 };
 
+// One workgroup's range of a tube: cells [lo, hi) of it.
+struct TubeSeg {
+    int tube, lo, hi;
+};
+
 // Batched 1D tubes (one persistent launch, one tube per workgroup at a time).
 struct TubeArgs {
     double *P[3];       // primitives P^n (in/out)
@@ -88,6 +93,10 @@ struct TubeArgs {
     const double *dt;   // per-tube dt
     const double *dx;   // per-tube dx
     unsigned int *queue;  // work counter
+    // k_tubes_split: state out, the workgroups' ranges and steps a launch
+    double *Pn[3], *Un[3];
+    const TubeSeg *seg;
+    int ksteps;
     int ntubes;
     int nsteps;
     int n_iter;

@@ -41,10 +41,6 @@ def HARM_HLL(P, N, dt, dx, T, eos, drops, rec, *kwargs, riemann="hll"):
     if N != P.size:
         raise ValueError("N must equal P.size")
     out = [P.copy()]
-    # one workgroup as wide as the tube (up to 1024 lanes): every stage is a
-    # single chunk with 4 waves per SIMD (1024-cell shock tube: 57 -> 23 ms
-    # against 128 lanes, the same bits)
-    block = min(1024, max(64, (N + 63) // 64 * 64))
     with Tubes([N], gamma=eos.gamma) as tb:
         tb.upload(P.arr1, P.arr2, P.arr3, [dt], [dx])
         tb.set_method(_rec_name(rec), riemann, n_iter, tol)
@@ -59,7 +55,7 @@ def HARM_HLL(P, N, dt, dx, T, eos, drops, rec, *kwargs, riemann="hll"):
                 k += 1
                 if t > thres:
                     break
-            tb.run(k, block=block, grid=1)
+            tb.run(k)
             if t > thres:
                 r, u, ux = tb.download()
                 q = ParVector1D(N)
