@@ -106,3 +106,30 @@ def test_tubes_split_over_workgroups(oracle, rec, riemann, lengths):
         got = np.stack(tb.download())
     want = _oracle_tubes(oracle, lengths, rho, u, ux, dt, dx, 5.0 / 3.0, rec, riemann, 23)
     assert np.array_equal(got, want, equal_nan=True)
+
+
+@pytest.mark.parametrize("rec,riemann", [("wenoz", "hll"), ("ppm", "hllc"), ("minmod", "hll")])
+@pytest.mark.parametrize("shape", [(4, 4, 4), (63, 8, 9), (64, 15, 6), (9, 16, 70), (5, 40), (130, 12)])
+def test_flux_regions(oracle, shape, rec, riemann):
+    """Fluxes of the kernel boundary around the sizes of its waves (63 faces
+    of a stream of rows; 8 columns of 7 faces): the oracle's bits on every
+    face of the region, nothing written outside it."""
+    from helpers import from_oracle3, to_oracle3
+    from verona_amd import DeviceGrid
+    progress(f"flux regions {shape} {rec} {riemann}")
+    nd = len(shape)
+    P = state3(*shape, seed=6) if nd == 3 else state2(*shape, seed=6)
+    Po = to_oracle3(P)
+    sl = (slice(None),) + (slice(2, -3),) * nd
+    mark = np.full(P.shape, 123.0, order="F")
+    with DeviceGrid(nd, *shape, *((1,) if nd == 2 else ()), gamma=G) as dev:
+        dev.upload("P", P)
+        for dim, slot in enumerate(["Fx", "Fy", "Fz"][:nd]):
+            dev.upload(slot, mark)
+            dev.fluxes(dim, 1e-7, rec, riemann)
+            a = dev.download(slot)
+            f = oracle.fluxes3 if nd == 3 else oracle.fluxes2
+            b = from_oracle3(f(Po, G, 1e-7, dim, rec, riemann))
+            assert np.array_equal(a[sl], b[sl])
+            a[sl] = 123.0
+            assert (a == 123.0).all()

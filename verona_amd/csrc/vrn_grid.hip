@@ -227,39 +227,128 @@ __global__ __launch_bounds__(256) void k_ref_limit(Geo G, double *P, double fl)
     }
 }
 
-// Fluxes: face i+1/2 along DIM for 0-based (i, j, k) in [2, N-3)^ndim; both
-// face states recomputed per face as in the reference (two reconstructions).
-template <int NV, int DIM, int REC, int RIEM>
-__global__ __launch_bounds__(256) void k_ref_fluxes(Geo G, const double *P, double *F, double g,
-                                                     double fl)
+// Fluxes: face i+1/2 along DIM for 0-based (i, j, k) in [2, N-3)^ndim.  With
+// PPM and WENO-Z each cell is reconstructed for both its faces at once (one
+// thread a face, both face states formed anew as in the reference, is twice
+// the reconstructions).  256^3, WENO-Z + HLL, x 918 -> 725 us, y and z 960 ->
+// 868 us; 160 x 144 x 128, PPM + HLLC, 225 -> 180 us a direction.  Bound by
+// the issue of the exact form's FP64 operations (the x sweep of the fused step
+// takes as long a cell); 80 B a cell take 275 us at 256^3 at the copy rate.
+template <int NV> __device__ __forceinline__ void ref_floor(double fl, double *p)
 {
-    const int ni = G.NX - 5, nj = G.NY - 5, nk = NV == 5 ? G.NZ - 5 : 1;
-    const long n = (long)ni * nj * nk;
-    const long sd = DIM == 0 ? 1 : (DIM == 1 ? (long)G.px : (long)G.px * G.NY);
-    for (long t = (long)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += (long)gridDim.x * blockDim.x) {
-        const int i = 2 + (int)(t % ni);
-        const long r = t / ni;
-        const int j = 2 + (int)(r % nj);
-        const int k = NV == 5 ? 2 + (int)(r / nj) : 0;
-        const long c = gidx(G, i, j, k);
-        double PL[NV], PR[NV];
+    p[0] = jmax(fl, p[0]);
+    p[1] = jmax(fl, p[1]);
+}
+
+// Value of lane l - 8 (lanes 0..7: any).
+__device__ __forceinline__ double shift_up8(double v)
+{
+    const int at = ((int)__lane_id() - 8) << 2;
+    const int lo = __builtin_amdgcn_ds_bpermute(at, __double2loint(v));
+    const int hi = __builtin_amdgcn_ds_bpermute(at, __double2hiint(v));
+    return __hiloint2double(hi, lo);
+}
+
+// y and z: a wave is 8 columns of 8 cells along DIM, overlapping the next
+// wave's by one; the upper state of the cell before comes from lane l - 8.
+// The 14 % of reconstructions that overlap cost less than the alternatives:
+// marching along a column holds 200 registers or more (870 us at 256^3 with
+// 16 faces a lane, but 55 us instead of 23 at 64^3), rows of waves that pass
+// states through LDS wait at their barrier (980 us).
+template <int NV, int DIM, int REC, int RIEM>
+__global__ __launch_bounds__(256) void k_ref_flux_yz(Geo G, const double *__restrict__ P, double *__restrict__ F, double g,
+                                                     double fl, unsigned groups)
+{
+    const int lane = threadIdx.x & 63, row = lane >> 3;
+    const unsigned wave = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (wave >= groups) return;
+    const unsigned ni = G.NX - 5, cols = ni * (NV == 5 ? (DIM == 1 ? G.NZ : G.NY) - 5 : 1), cg = (cols + 7) / 8;
+    const int Nd = DIM == 1 ? G.NY : G.NZ;
+    const unsigned wr = wave / cg, col = (wave - wr * cg) * 8 + (lane & 7), t = min(col, cols - 1), o = t / ni;
+    const int m = 2 + (int)wr * 7 + row, mc = min(m, Nd - 3);
+    const int x = 2 + (int)(t - o * ni);
+    const long sd = DIM == 1 ? (long)G.px : (long)G.px * G.NY;
+    const long ps = G.ps;
+    const long b = DIM == 1 ? gidx(G, x, mc, NV == 5 ? 2 + o : 0) : gidx(G, x, 2 + o, mc);
+    double lo[NV], up[NV], upl[NV];
 #pragma unroll
-        for (int v = 0; v < NV; v++) {
-            const double *q = P + v * G.ps + c;
-            double lo, hi;
-            recon<REC>(q[-2 * sd], q[-sd], q[0], q[sd], q[2 * sd], lo, hi);
-            PL[v] = hi;
-            recon<REC>(q[-sd], q[0], q[sd], q[2 * sd], q[3 * sd], lo, hi);
-            PR[v] = lo;
-        }
-        PL[0] = jmax(fl, PL[0]);
-        PR[0] = jmax(fl, PR[0]);
-        PL[1] = jmax(fl, PL[1]);
-        PR[1] = jmax(fl, PR[1]);
-        double Fo[NV];
-        face_flux<NV, DIM, RIEM>(PL, PR, g, Fo);
+    for (int v = 0; v < NV; v++) {
+        const double *q = P + v * ps + b;
+        recon<REC>(q[-2 * sd], q[-sd], q[0], q[sd], q[2 * sd], lo[v], up[v]);
+    }
+    ref_floor<NV>(fl, lo);
+    ref_floor<NV>(fl, up);
 #pragma unroll
-        for (int v = 0; v < NV; v++) F[v * G.ps + c] = Fo[v];
+    for (int v = 0; v < NV; v++) upl[v] = shift_up8(up[v]);
+    double Fo[NV];
+    face_flux<NV, DIM, RIEM>(upl, lo, g, Fo);
+    if (row > 0 && m <= Nd - 3 && col < cols) {
+#pragma unroll
+        for (int v = 0; v < NV; v++) F[v * ps + b - sd] = Fo[v];
+    }
+}
+
+// y and z with minmod, whose reconstruction is cheap: a thread a face, two
+// reconstructions, whole lines of x (104 us at 160 x 144 x 128; 118 us by
+// k_ref_flux_yz, whose 64-byte rows are what it waits for then).
+template <int NV, int DIM, int REC, int RIEM>
+__global__ __launch_bounds__(256) void k_ref_flux_face(Geo G, const double *__restrict__ P, double *__restrict__ F,
+                                                       double g, double fl)
+{
+    const unsigned ni = G.NX - 5, nj = G.NY - 5, n = ni * nj * (NV == 5 ? G.NZ - 5 : 1);
+    const unsigned t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= n) return;
+    const unsigned r = t / ni, k = r / nj;
+    const long sd = DIM == 1 ? (long)G.px : (long)G.px * G.NY;
+    const long b = gidx(G, 2 + (int)(t - r * ni), 2 + (int)(r - k * nj), NV == 5 ? 2 + (int)k : 0);
+    double PL[NV], PR[NV];
+#pragma unroll
+    for (int v = 0; v < NV; v++) {
+        const double *q = P + v * G.ps + b;
+        double lo, hi;
+        recon<REC>(0.0, q[-sd], q[0], q[sd], 0.0, lo, hi);
+        PL[v] = hi;
+        recon<REC>(0.0, q[0], q[sd], q[2 * sd], 0.0, lo, hi);
+        PR[v] = lo;
+    }
+    ref_floor<NV>(fl, PL);
+    ref_floor<NV>(fl, PR);
+    double Fo[NV];
+    face_flux<NV, DIM, RIEM>(PL, PR, g, Fo);
+#pragma unroll
+    for (int v = 0; v < NV; v++) F[v * G.ps + b] = Fo[v];
+}
+
+// x: the cells 2 .. NX-3 of all rows are one stream, of which a wave takes 64
+// that overlap the next wave's by one: the left cell's upper state comes from
+// the lane to the left, and nothing else is shared.
+template <int NV, int REC, int RIEM>
+__global__ __launch_bounds__(256) void k_ref_flux_x(Geo G, const double *__restrict__ P, double *__restrict__ F, double g,
+                                                    double fl)
+{
+    const int lane = threadIdx.x & 63;
+    const unsigned wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
+    const unsigned E = G.NX - 4, nj = G.NY - 5;
+    const unsigned total = E * nj * (NV == 5 ? G.NZ - 5 : 1);
+    const unsigned t = min(wave * 63 + lane, total - 1);
+    const unsigned r = t / E, cc = t - r * E, k = r / nj;
+    const long b = gidx(G, 2 + cc, 2 + (r - k * nj), NV == 5 ? 2 + k : 0);
+    const long ps = G.ps;
+    double lo[NV], up[NV], upl[NV];
+#pragma unroll
+    for (int v = 0; v < NV; v++) {
+        const double *q = P + v * ps + b;
+        recon<REC>(q[-2], q[-1], q[0], q[1], q[2], lo[v], up[v]);
+    }
+    ref_floor<NV>(fl, lo);
+    ref_floor<NV>(fl, up);
+#pragma unroll
+    for (int v = 0; v < NV; v++) upl[v] = shift_up1(up[v], up[v]);
+    double Fo[NV];
+    face_flux<NV, 0, RIEM>(upl, lo, g, Fo);
+    if (lane >= 1 && cc >= 1 && wave * 63 + lane < total) {
+#pragma unroll
+        for (int v = 0; v < NV; v++) F[v * ps + b - 1] = Fo[v];
     }
 }
 
@@ -853,23 +942,36 @@ int vrn_limit(vrn_ctx *c, double floor_)
 
 }  // extern "C"
 
-template <int NV, int DIM>
-static void launch_ref_flux(vrn_ctx *c, int rec, int riem, double fl)
+template <int NV, int DIM, int REC, int RIEM> static void launch_ref_flux(vrn_ctx *c, double fl)
 {
     const Geo &G = c->G;
-    long n = (long)(G.NX - 5) * (G.NY - 5) * (NV == 5 ? G.NZ - 5 : 1);
-    dim3 gb(grid_blocks(n, 256)), bb(256);
-    double *F = c->F[DIM];
-#define VRN_FL(R_, M_) hipLaunchKernelGGL((k_ref_fluxes<NV, DIM, R_, M_>), gb, bb, 0, c->s, G, c->P, F, c->gamma, fl)
-    if (riem == VRN_RIEMANN_HLL) {
-        if (rec == VRN_REC_WENOZ) VRN_FL(REC_WENOZ, RIEM_HLL);
-        else if (rec == VRN_REC_PPM) VRN_FL(REC_PPM, RIEM_HLL);
-        else VRN_FL(REC_MINMOD, RIEM_HLL);
+    if constexpr (DIM == 0) {
+        const long n = (long)(G.NX - 4) * (G.NY - 5) * (NV == 5 ? G.NZ - 5 : 1);
+        const long waves = (n + 62) / 63;
+        hipLaunchKernelGGL((k_ref_flux_x<NV, REC, RIEM>), dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, c->s, G, c->P,
+                           c->F[0], c->gamma, fl);
+    } else if constexpr (REC == REC_MINMOD) {
+        const long n = (long)(G.NX - 5) * (G.NY - 5) * (NV == 5 ? G.NZ - 5 : 1);
+        hipLaunchKernelGGL((k_ref_flux_face<NV, DIM, REC, RIEM>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, c->s, G,
+                           c->P, c->F[DIM], c->gamma, fl);
     } else {
-        if (rec == VRN_REC_WENOZ) VRN_FL(REC_WENOZ, RIEM_HLLC);
-        else if (rec == VRN_REC_PPM) VRN_FL(REC_PPM, RIEM_HLLC);
-        else VRN_FL(REC_MINMOD, RIEM_HLLC);
+        const long cols = (long)(G.NX - 5) * (NV == 5 ? (DIM == 1 ? G.NZ : G.NY) - 5 : 1);
+        const long L = (DIM == 1 ? G.NY : G.NZ) - 5, groups = (cols + 7) / 8 * ((L + 6) / 7);
+        hipLaunchKernelGGL((k_ref_flux_yz<NV, DIM, REC, RIEM>), dim3((unsigned)((groups + 3) / 4)), dim3(256), 0, c->s, G,
+                           c->P, c->F[DIM], c->gamma, fl, (unsigned)groups);
     }
+}
+
+template <int NV, int DIM> static void launch_ref_flux(vrn_ctx *c, int rec, int riem, double fl)
+{
+#define VRN_FL(M_)                                                            \
+    do {                                                                      \
+        if (rec == VRN_REC_WENOZ) launch_ref_flux<NV, DIM, REC_WENOZ, M_>(c, fl); \
+        else if (rec == VRN_REC_PPM) launch_ref_flux<NV, DIM, REC_PPM, M_>(c, fl); \
+        else launch_ref_flux<NV, DIM, REC_MINMOD, M_>(c, fl);                 \
+    } while (0)
+    if (riem == VRN_RIEMANN_HLL) VRN_FL(RIEM_HLL);
+    else VRN_FL(RIEM_HLLC);
 #undef VRN_FL
 }
 
