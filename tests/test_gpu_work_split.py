@@ -133,3 +133,32 @@ def test_flux_regions(oracle, shape, rec, riemann):
             assert np.array_equal(a[sl], b[sl])
             a[sl] = 123.0
             assert (a == 123.0).all()
+
+
+def test_large_copies_from_two_threads():
+    """Copies large enough for the pinned staging (and the ragged last slice
+    of one), repeated, from two threads that want it at once, into fresh and
+    into used arrays: every byte arrives."""
+    import threading
+
+    from verona_amd import DeviceGrid
+    progress("large copies")
+    errors = []
+
+    def go(seed, n):
+        rng = np.random.default_rng(seed)
+        P = np.asfortranarray(rng.standard_normal((5, n + 6, n + 5, n + 7)))
+        with DeviceGrid(3, n, n - 1, n + 1, gamma=G) as dev:
+            out = np.empty(P.shape, order="F")
+            for k in range(4):
+                P[:, k, :, :] += 1.0
+                dev.upload("U", P)
+                dev.download("U", out=out)
+                if not (np.array_equal(out, P) and np.array_equal(dev.download("U"), P)):
+                    errors.append((seed, k))
+    threads = [threading.Thread(target=go, args=a) for a in ((1, 95), (2, 90), (3, 61))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors

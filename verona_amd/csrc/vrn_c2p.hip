@@ -33,6 +33,7 @@
 #include "../../include/verona_c2p.h"
 #define VRN_NS vrn_c4
 #include "vrn_physics.hpp"
+#include "vrn_xfer.hpp"
 
 #include <hip/hip_runtime.h>
 
@@ -1015,6 +1016,7 @@ constexpr int MAX_SOLVE_GRID = 4096;
 }  // namespace
 
 struct vrn_c2p {
+    vrn_xfer::Hold hold;
     long n_max = 0, n = 0;
     double g = 0;
     hipStream_t s = nullptr;
@@ -1180,7 +1182,7 @@ int vrn_c2p_upload(vrn_c2p *h, int64_t n, const double *U, const double *P_prev)
     if (!h || !U) return fail(-1, "vrn_c2p_upload: NULL argument");
     if (n < 1 || n > h->n_max) return fail(-1, "vrn_c2p_upload: n = %lld outside [1, %ld]", (long long)n, h->n_max);
     const size_t nb = sizeof(double) * 5 * (size_t)n;
-    HIPCHK(hipMemcpyAsync(h->stage, U, nb, hipMemcpyHostToDevice, h->s));
+    HIPCHK(vrn_xfer::h2d(h->stage, U, nb, h->s));
     hipLaunchKernelGGL(k_aos_to_soa, dim3(grid_for(5 * n, 256)), dim3(256), 0, h->s, (long)n,
                        (const double *)h->stage, h->U);
     HIPCHK(hipGetLastError());
@@ -1188,7 +1190,7 @@ int vrn_c2p_upload(vrn_c2p *h, int64_t n, const double *U, const double *P_prev)
     if (P_prev) {
         if (!h->Pprev) HIPCHK(hipMalloc(&h->Pprev, sizeof(double) * 5 * (size_t)h->n_max));
         HIPCHK(hipStreamSynchronize(h->s));
-        HIPCHK(hipMemcpyAsync(h->stage, P_prev, nb, hipMemcpyHostToDevice, h->s));
+        HIPCHK(vrn_xfer::h2d(h->stage, P_prev, nb, h->s));
         hipLaunchKernelGGL(k_aos_to_soa, dim3(grid_for(5 * n, 256)), dim3(256), 0, h->s, (long)n,
                            (const double *)h->stage, h->Pprev);
         HIPCHK(hipGetLastError());
@@ -1294,9 +1296,9 @@ int vrn_c2p_download(vrn_c2p *h, double *P, double *W0, uint8_t *iters)
         hipLaunchKernelGGL(k_soa_to_aos, dim3(grid_for(5 * n, 256)), dim3(256), 0, h->s, n, (const double *)h->P,
                            h->stage);
         HIPCHK(hipGetLastError());
-        HIPCHK(hipMemcpyAsync(P, h->stage, sizeof(double) * 5 * (size_t)n, hipMemcpyDeviceToHost, h->s));
+        HIPCHK(vrn_xfer::d2h(P, h->stage, sizeof(double) * 5 * (size_t)n, h->s));
     }
-    if (W0) HIPCHK(hipMemcpyAsync(W0, h->W0, sizeof(double) * (size_t)n, hipMemcpyDeviceToHost, h->s));
+    if (W0) HIPCHK(vrn_xfer::d2h(W0, h->W0, sizeof(double) * (size_t)n, h->s));
     if (iters) HIPCHK(hipMemcpyAsync(iters, h->iters, (size_t)n, hipMemcpyDeviceToHost, h->s));
     HIPCHK(hipStreamSynchronize(h->s));
     return 0;
@@ -1329,13 +1331,13 @@ int vrn_mlp_features(vrn_c2p *h, int64_t n, const double *U, const double *P, fl
     if (!h || !U || !X || !valid || (P && !T)) return fail(-1, "vrn_mlp_features: NULL argument");
     if (n < 1 || n > h->n_max) return fail(-1, "vrn_mlp_features: n = %lld out of range", (long long)n);
     if (int rc = ensure_pairs(h, n)) return rc;
-    HIPCHK(hipMemcpyAsync(h->pairU, U, sizeof(double) * 5 * (size_t)n, hipMemcpyHostToDevice, h->s));
-    if (P) HIPCHK(hipMemcpyAsync(h->pairP, P, sizeof(double) * 5 * (size_t)n, hipMemcpyHostToDevice, h->s));
+    HIPCHK(vrn_xfer::h2d(h->pairU, U, sizeof(double) * 5 * (size_t)n, h->s));
+    if (P) HIPCHK(vrn_xfer::h2d(h->pairP, P, sizeof(double) * 5 * (size_t)n, h->s));
     hipLaunchKernelGGL(k_features, dim3(grid_for(n, 256)), dim3(256), 0, h->s, (long)n, (const double *)h->pairU,
                        P ? (const double *)h->pairP : (const double *)nullptr, h->g, h->X, h->T, h->valid);
     HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(X, h->X, sizeof(float) * NIN * (size_t)n, hipMemcpyDeviceToHost, h->s));
-    if (P) HIPCHK(hipMemcpyAsync(T, h->T, sizeof(float) * 2 * (size_t)n, hipMemcpyDeviceToHost, h->s));
+    HIPCHK(vrn_xfer::d2h(X, h->X, sizeof(float) * NIN * (size_t)n, h->s));
+    if (P) HIPCHK(vrn_xfer::d2h(T, h->T, sizeof(float) * 2 * (size_t)n, h->s));
     HIPCHK(hipMemcpyAsync(valid, h->valid, (size_t)n, hipMemcpyDeviceToHost, h->s));
     HIPCHK(hipStreamSynchronize(h->s));
     return 0;
@@ -1348,12 +1350,12 @@ int vrn_mlp_infer(vrn_c2p *h, int64_t n, const float *X, float *Y)
     if (!h->have_params) return fail(-1, "vrn_mlp_infer: no parameters set or trained");
     if (int rc = ensure_pairs(h, n)) return rc;
     if (int rc = ensure_net(h)) return rc;
-    HIPCHK(hipMemcpyAsync(h->X, X, sizeof(float) * NIN * (size_t)n, hipMemcpyHostToDevice, h->s));
+    HIPCHK(vrn_xfer::h2d(h->X, X, sizeof(float) * NIN * (size_t)n, h->s));
     const long nchunks = (n + 63) / 64;
     hipLaunchKernelGGL(k_infer, dim3(grid_for(nchunks, 4, 4096)), dim3(256), 0, h->s, (long)n, (const float *)h->X,
                        (const NetRegs *)h->net, h->T);
     HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(Y, h->T, sizeof(float) * 2 * (size_t)n, hipMemcpyDeviceToHost, h->s));
+    HIPCHK(vrn_xfer::d2h(Y, h->T, sizeof(float) * 2 * (size_t)n, h->s));
     HIPCHK(hipStreamSynchronize(h->s));
     return 0;
 }
@@ -1365,7 +1367,7 @@ int vrn_mlp_grad(vrn_c2p *h, int64_t n, const float *X, const float *T, const fl
     if (n < 1 || n > MAX_BATCH) return fail(-1, "vrn_mlp_grad: n = %lld outside [1, %d]", (long long)n, MAX_BATCH);
     if (int rc = ensure_train(h)) return rc;
     if (int rc = ensure_pairs(h, n)) return rc;
-    HIPCHK(hipMemcpyAsync(h->X, X, sizeof(float) * NIN * (size_t)n, hipMemcpyHostToDevice, h->s));
+    HIPCHK(vrn_xfer::h2d(h->X, X, sizeof(float) * NIN * (size_t)n, h->s));
     HIPCHK(hipMemcpyAsync(h->T, T, sizeof(float) * 2 * (size_t)n, hipMemcpyHostToDevice, h->s));
     HIPCHK(hipMemcpyAsync(h->train[0]->prm, params, sizeof(float) * NPARAM, hipMemcpyHostToDevice, h->s));
     TrainArgs ta{};
@@ -1400,8 +1402,8 @@ int vrn_mlp_train(vrn_c2p *h, int64_t n, const double *U, const double *P, const
     if (int rc = ensure_train(h)) return rc;
     if (int rc = ensure_pairs(h, n)) return rc;
     HIPCHK(hipEventRecord(h->e0, h->s));
-    HIPCHK(hipMemcpyAsync(h->pairU, U, sizeof(double) * 5 * (size_t)n, hipMemcpyHostToDevice, h->s));
-    HIPCHK(hipMemcpyAsync(h->pairP, P, sizeof(double) * 5 * (size_t)n, hipMemcpyHostToDevice, h->s));
+    HIPCHK(vrn_xfer::h2d(h->pairU, U, sizeof(double) * 5 * (size_t)n, h->s));
+    HIPCHK(vrn_xfer::h2d(h->pairP, P, sizeof(double) * 5 * (size_t)n, h->s));
     hipLaunchKernelGGL(k_features, dim3(grid_for(n, 256)), dim3(256), 0, h->s, (long)n, (const double *)h->pairU,
                        (const double *)h->pairP, h->g, h->X, h->T, h->valid);
     HIPCHK(hipGetLastError());

@@ -26,6 +26,7 @@
 //    unconverged go to a rescue list finished by the full cascade.
 #include "../../include/verona_hip.h"
 #include "vrn_types.hpp"
+#include "vrn_xfer.hpp"
 #define VRN_NS vrn
 #include "vrn_physics.hpp"
 #include "vrn_sweeps.hpp"
@@ -480,6 +481,7 @@ enum { KN_X, KN_Y, KN_ZC, KN_F2D, KN_RESCUE, KN_GHOST, KN_CFL, KN_FLUX, KN_UPD, 
 }  // namespace
 
 struct vrn_ctx {
+    vrn_xfer::Hold hold;
     int ndim = 3, NV = 5;
     Geo G{};
     double gamma = 4.0 / 3.0;
@@ -853,7 +855,7 @@ int vrn_upload(vrn_ctx *c, int slot, const double *host)
     if (!d || !host) return fail(VRN_E_ARG, "bad slot %d or null host pointer", slot);
     const Geo &G = c->G;
     size_t bytes = sizeof(double) * (size_t)c->NV * G.NX * G.NY * G.NZ;
-    HIPCHK(hipMemcpyAsync(c->stg, host, bytes, hipMemcpyHostToDevice, c->s));
+    HIPCHK(vrn_xfer::h2d(c->stg, host, bytes, c->s));
     long n = (long)G.NX * G.NY * G.NZ;
     if (c->NV == 5)
         hipLaunchKernelGGL(k_aos_to_soa<5>, dim3(grid_blocks(n, 256)), dim3(256), 0, c->s, G, c->stg, d);
@@ -884,8 +886,7 @@ int vrn_download(vrn_ctx *c, int slot, double *host)
     else
         hipLaunchKernelGGL(k_soa_to_aos<4>, dim3(grid_blocks(n, 256)), dim3(256), 0, c->s, G, d, c->stg);
     HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(host, c->stg, sizeof(double) * (size_t)c->NV * n, hipMemcpyDeviceToHost, c->s));
-    HIPCHK(hipStreamSynchronize(c->s));
+    HIPCHK(vrn_xfer::d2h(host, c->stg, sizeof(double) * (size_t)c->NV * n, c->s));
     return 0;
 }
 

@@ -22,6 +22,7 @@
 // in vrn_tubes_fast.hip (vrn_tubes_set_precision selects one).
 #include "../../include/verona_hip.h"
 #include "vrn_tubes_kern.hpp"
+#include "vrn_xfer.hpp"
 
 #include <hip/hip_runtime.h>
 
@@ -59,6 +60,7 @@ int tfail(int code, const char *fmt, ...)
 }  // namespace
 
 struct vrn_tubes {
+    vrn_xfer::Hold hold;
     int ntubes = 0;
     long ncell = 0;
     double gamma = 5.0 / 3.0;
@@ -232,8 +234,8 @@ int vrn_tubes_upload(vrn_tubes *c, const double *rho, const double *u, const dou
     const size_t b = sizeof(double) * c->ncell;
     const double *src[3] = {rho, u, ux};
     for (int v = 0; v < 3; v++) {
-        TCHK(hipMemcpyAsync(c->args.P[v], src[v], b, hipMemcpyHostToDevice, c->s));
-        TCHK(hipMemcpyAsync((void *)c->args.P0[v], src[v], b, hipMemcpyHostToDevice, c->s));
+        TCHK(vrn_xfer::h2d(c->args.P[v], src[v], b, c->s));
+        TCHK(hipMemcpyAsync((void *)c->args.P0[v], c->args.P[v], b, hipMemcpyDeviceToDevice, c->s));
     }
     TCHK(hipMemcpyAsync(c->dt, dt, sizeof(double) * c->ntubes, hipMemcpyHostToDevice, c->s));
     TCHK(hipMemcpyAsync(c->dx, dx, sizeof(double) * c->ntubes, hipMemcpyHostToDevice, c->s));
@@ -248,8 +250,7 @@ int vrn_tubes_download(vrn_tubes *c, double *rho, double *u, double *ux)
     if (!c || !rho || !u || !ux) return tfail(VRN_E_ARG, "null argument");
     const size_t b = sizeof(double) * c->ncell;
     double *dst[3] = {rho, u, ux};
-    for (int v = 0; v < 3; v++) TCHK(hipMemcpyAsync(dst[v], c->args.P[v], b, hipMemcpyDeviceToHost, c->s));
-    TCHK(hipStreamSynchronize(c->s));
+    for (int v = 0; v < 3; v++) TCHK(vrn_xfer::d2h(dst[v], c->args.P[v], b, c->s));
     return 0;
 }
 
