@@ -193,12 +193,12 @@ int vrn_timing_report(vrn_ctx *ctx, char *names, int name_len, int64_t *counts, 
 int vrn_set_partition(vrn_ctx *ctx, int rows_per_wave, int xseg, int seg_len);
 int vrn_get_partition(vrn_ctx *ctx, int *rows_per_wave, int *xseg, int *seg_len);
 
-/* 3D, VRN_PREC_FP64 and VRN_PREC_FP64_FAST: whether the x direction runs
- * inside the y march (on = 1, the default) or as its own sweep (0).  No
- * counterpart in the reference and no change of arithmetic: both solve the
- * same faces and apply the same updates in the same order, bit for bit; the
- * fused form moves 116 B less per cell and stage.  The FP32 form and 2D
- * always use the separate x sweep. */
+/* VRN_PREC_FP64 and VRN_PREC_FP64_FAST: whether the x direction runs inside
+ * the y march (on = 1, the default) or as its own sweep (0).  No counterpart
+ * in the reference and no change of arithmetic: both solve the same faces and
+ * apply the same updates in the same order, bit for bit; in 3D the fused form
+ * moves 116 B less per cell and stage.  The FP32 form always uses the separate
+ * x sweep, and so does the 2D exact form with PPM and minmod. */
 int vrn_set_xy_fusion(vrn_ctx *ctx, int on);
 
 

@@ -162,3 +162,30 @@ def test_large_copies_from_two_threads():
     for t in threads:
         t.join()
     assert not errors
+
+
+@pytest.mark.parametrize("form", ["fp64", "fp64fast"])
+@pytest.mark.parametrize("rec,riemann", [("wenoz", "hllc"), ("ppm", "hll"), ("minmod", "hllc")])
+@pytest.mark.parametrize("shape,kind", [((4, 5), "periodic"), ((63, 9), "outflow"), ((64, 20), "none"), ((66, 17), "outflow"),
+                                        ((131, 40), "periodic")])
+def test_x_inside_the_2d_march(shape, kind, rec, riemann, form):
+    """2D: the x direction inside the y march gives the bits of its own sweep,
+    ghost cells included, around the widths of a wave."""
+    from verona_amd import DeviceGrid
+    progress(f"2D x-y march {shape} {kind} {rec} {riemann} {form}")
+    P = state2(*shape, seed=8)
+    bc = (kind,) * 4 + ("none",) * 2
+    outs = []
+    for on in (True, False):
+        with DeviceGrid(2, *shape, gamma=G) as dev:
+            dev.set_xy_fusion(on)
+            dev.upload("P", P)
+            dev.fill_ghosts(bc)
+            dev.prim_to_cons()
+            dev.set_step(ref_mode=False, rec=rec, riemann=riemann, integrator="rk3", precision=form, n_iter=50, tol=1e-10,
+                         floor=1e-7, cfl=0.3, dx=1 / shape[0], dy=1 / shape[1], bc=bc)
+            for _ in range(3):
+                dev.step()
+            outs.append((dev.download("P"), dev.download("U")))
+    for a, b in zip(*outs):
+        assert np.array_equal(a, b, equal_nan=True)

@@ -383,12 +383,12 @@ __global__ __launch_bounds__(256, VRN_MARCH_MIN_WAVES) void k_march(SweepArgs a)
 {
     // lanes per block: 256 in 3D (four o-rows of 64 columns), 64 in 2D
     constexpr int WS = NV == 5 ? 256 : 64;
-    // XY (3D y march only): the march also does the x direction of each row
+    // XY (y march only): the march also does the x direction of each row
     // it updates, with the ring row of its 64 columns as the x stencils.  The
     // six faces at a wave's ends whose stencils leave those columns (three
     // each side) are solved every 8 rows for the next 8 by the whole wave
     // (edge_faces) into eb[row & 7][wave][face][var].
-    static_assert(!XY || (DIM == 1 && NV == 5 && !LAST), "x-y fusion is the 3D y march");
+    static_assert(!XY || (DIM == 1 && (NV == 4 || !LAST)), "x-y fusion is the y march");
     constexpr int WSR = WS;  // ring stride per (slot, variable)
     __shared__ R win[5 * NV * WSR];
     constexpr int EBR = (WS / 64) * 6 * NV;  // edge-face buffer stride per row
@@ -536,7 +536,7 @@ __global__ __launch_bounds__(256, VRN_MARCH_MIN_WAVES) void k_march(SweepArgs a)
                     }
                     // every 8 rows: the edge faces of rows c-1 .. c+6
                     if (((c - 1 - m0) & 7) == 0) {
-                        edge_faces<NV, R, REC, RIEM>(a, G, eb + wv * 6 * NV, EBR, lane, x0, xr, o, c - 1,
+                        edge_faces<NV, R, REC, RIEM>(a, G, eb + wv * 6 * NV, EBR, lane, x0, xr, NV == 5 ? o : 0, c - 1,
                                                      min(c + 7, m1), m0);
                         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
                         __builtin_amdgcn_wave_barrier();
@@ -681,27 +681,45 @@ __global__ __launch_bounds__(64) void k_rescue(SweepArgs a)
 }
 
 
+// Whether the 2D y march is the last sweep (RK combination, closed-form 4x4
+// Newton, Limit and rate inside the march; the separate pass gives the same
+// bits).
+#if defined(VRN_FAST)
+template <class R> constexpr bool fused_end2d() { return std::is_same<R, double>::value; }
+#else
+template <class R> constexpr bool fused_end2d() { return false; }
+#endif
+
 // Launch the three sweeps + rescue of one RK stage.
 template <int NV, class R, int REC, int RIEM>
 void launch_stage(hipStream_t s, const SweepArgs &a, const double dxs[3], void (*timer)(void *, int, int), void *tctx)
 {
     const Geo &G = a.geo;
     const int nxb = (G.NX - 6 + 63) / 64;
-    // 3D FP64 forms: the x direction runs inside the y march, which saves
-    // the x sweep's write and the y sweep's re-read of the accumulated U and
-    // one read of P per stage; the same fluxes and updates in the same
-    // order as the x and y sweeps.
-    const bool fxy = NV == 5 && std::is_same<R, double>::value && a.fuse_xy;
+    // FP64 forms: the x direction runs inside the y march, which saves the x
+    // sweep's write and the y sweep's re-read of the accumulated U and one
+    // read of P per stage; the same fluxes and updates in the same order as
+    // the x and y sweeps.  In 2D the fast form's stage is then one kernel
+    // (fused / split, us a stage: 2048^2 WENO-Z 282 / 300, PPM 364 / 440,
+    // minmod 204 / 241; 512^2 WENO-Z 35 / 51); the exact form gains with
+    // WENO-Z (1024^2 105 / 129, 2048^2 366 / 377) and not with the others
+    // (2048^2 PPM 583 / 546, minmod 244 / 233), whose selects already fill
+    // the march.
+    const bool fxy = std::is_same<R, double>::value && (NV == 5 || fused_end2d<R>() || REC == REC_WENOZ) && a.fuse_xy;
     if (fxy) {
-        if constexpr (NV == 5 && std::is_same<R, double>::value) {
+        if constexpr (std::is_same<R, double>::value) {
             SweepArgs ay = a;
             ay.dx_dim = dxs[1];
             ay.dx_x = dxs[0];
             ay.seg_len = a.seg_y;
-            int nseg = (G.NY - 6 + a.seg_y - 1) / a.seg_y;
+            const int nseg = (G.NY - 6 + a.seg_y - 1) / a.seg_y;
             timer(tctx, 10, 0);
-            hipLaunchKernelGGL((k_march<5, 1, R, REC, RIEM, false, true>), dim3(nxb, (G.NZ - 6 + 3) / 4, nseg),
-                               dim3(256), 0, s, ay);
+            if constexpr (NV == 5)
+                hipLaunchKernelGGL((k_march<5, 1, R, REC, RIEM, false, true>), dim3(nxb, (G.NZ - 6 + 3) / 4, nseg),
+                                   dim3(256), 0, s, ay);
+            else
+                hipLaunchKernelGGL((k_march<4, 1, R, REC, RIEM, fused_end2d<R>(), true>), dim3(nxb, 1, nseg), dim3(64), 0,
+                                   s, ay);
             timer(tctx, 10, 1);
         }
     } else {
@@ -738,22 +756,16 @@ void launch_stage(hipStream_t s, const SweepArgs &a, const double dxs[3], void (
             timer(tctx, 4, 1);
         }
     } else {
-        SweepArgs ay = a;
-        ay.dx_dim = dxs[1];
-        ay.seg_len = a.seg_y;
-        int nseg = (G.NY - 6 + a.seg_y - 1) / a.seg_y;
-#if defined(VRN_FAST)
-        // fast FP64 form: the y sweep is the last sweep (RK combination,
-        // closed-form 4x4 Newton, Limit and rate inside the march); same
-        // results as the separate pass, bit for bit
-        timer(tctx, 1, 0);
-        hipLaunchKernelGGL((k_march<4, 1, R, REC, RIEM, true>), dim3(nxb, 1, nseg), dim3(64), 0, s, ay);
-        timer(tctx, 1, 1);
-        return;
-#endif
-        timer(tctx, 1, 0);
-        hipLaunchKernelGGL((k_march<4, 1, R, REC, RIEM, false>), dim3(nxb, 1, nseg), dim3(64), 0, s, ay);
-        timer(tctx, 1, 1);
+        if (!fxy) {
+            SweepArgs ay = a;
+            ay.dx_dim = dxs[1];
+            ay.seg_len = a.seg_y;
+            timer(tctx, 1, 0);
+            hipLaunchKernelGGL((k_march<4, 1, R, REC, RIEM, fused_end2d<R>()>),
+                               dim3(nxb, 1, (G.NY - 6 + a.seg_y - 1) / a.seg_y), dim3(64), 0, s, ay);
+            timer(tctx, 1, 1);
+        }
+        if (fused_end2d<R>()) return;
         // about 2048 blocks of 256 lanes: x columns of 256 cells by row groups
         const int bx = (G.NX - 6 + 255) / 256;
         const int by = std::max(1, std::min(G.NY - 6, 2048 / bx));
