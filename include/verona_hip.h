@@ -168,8 +168,9 @@ typedef struct {
  * both x faces the ghost fill leaves P's x faces to be filled by the next
  * entry point that reads P's ghost cells (the fused kernel reads them
  * through the rules), so callers always see complete ghost cells.
- * *dt_used (may be NULL) receives the step's dt; in CFL mode that costs one
- * small device-to-host read. */
+ * *dt_used (may be NULL) receives the step's dt; in CFL mode the call then
+ * waits until the GPU has begun the step (its dt is formed first), not for the
+ * step itself. */
 int vrn_step(vrn_ctx *ctx, const vrn_step_params *p, double *dt_used);
 
 /* Per-kernel timing with HIP events on the context's stream.  enable = 1:
