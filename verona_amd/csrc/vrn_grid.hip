@@ -752,9 +752,11 @@ static void partition_sweeps(vrn_ctx *c)
         if (c->xseg > 1) c->rows_per_wave = 1;
     }
     for (int f = 0; f < 2; f++) {
+        // the x-y march (FP64) takes rows of 64 cells, the others any 256 columns
         const int nxb = (Nxi + 63) / 64;
-        c->seg_y[f] = march_segment(c->ndim, f == 1, Nyi, nxb * (c->ndim == 3 ? (Nzi + 3) / 4 : 1));
-        c->seg_z[f] = march_segment(c->ndim, f == 1, Nzi, nxb * ((Nyi + 3) / 4));
+        c->seg_y[f] = march_segment(c->ndim, f == 1, Nyi,
+                                    c->ndim == 2 ? nxb : (f ? (int)march_blocks(c->G, 1) : nxb * ((Nzi + 3) / 4)));
+        if (c->ndim == 3) c->seg_z[f] = march_segment(3, f == 1, Nzi, (int)march_blocks(c->G, 2));
     }
 }
 

@@ -404,15 +404,21 @@ __global__ __launch_bounds__(256, VRN_MARCH_MIN_WAVES) void k_march(SweepArgs a)
     __shared__ R curv[CARRY ? 2 * NV * WS : 1];
     const Geo G = a.geo;
     const int tid = threadIdx.x;
-    const int x = 3 + blockIdx.x * 64 + (threadIdx.x & 63);
-    const int o = 3 + blockIdx.y * (blockDim.x >> 6) + (threadIdx.x >> 6);
     const int Nd = DIM == 1 ? G.NY : G.NZ;
     const int No = NV == 5 ? (DIM == 1 ? G.NZ : G.NY) : 7;
+    // the block's columns: 256 consecutive ones of all (x, o), x fastest, so
+    // that only the last block has idle lanes whatever the width (161 cells by
+    // rows of 64 idle 16 % of them); the x-y march needs whole rows of 64
+    constexpr bool PACK = NV == 5 && !XY;
+    const unsigned pt = blockIdx.x * 256 + threadIdx.x, pr = PACK ? pt / (unsigned)(G.NX - 6) : 0;
+    const int x = PACK ? 3 + (int)(pt - pr * (unsigned)(G.NX - 6)) : 3 + blockIdx.x * 64 + (threadIdx.x & 63);
+    int o = PACK ? 3 + (int)pr : 3 + blockIdx.y * (blockDim.x >> 6) + (threadIdx.x >> 6);
     const int m0 = 3 + blockIdx.z * a.seg_len;
     // whole-wave exits only: a partially active wave keeps all lanes for the
     // cross-lane reductions and masks the inactive ones.
-    if (o >= No - 3 || m0 >= Nd - 3) return;
-    const bool act = x < G.NX - 3;
+    const bool act = PACK ? o < No - 3 : x < G.NX - 3;
+    if ((PACK ? !__any(act) : o >= No - 3) || m0 >= Nd - 3) return;
+    if (PACK && !act) o = 3;
     // XY: every lane holds its own column (inactive lanes a ghost or the
     // last one), since the x stencils of the active lanes reach into them;
     // ghost columns through the x boundary rules when the last ghost pass
@@ -687,6 +693,12 @@ __global__ __launch_bounds__(64) void k_rescue(SweepArgs a)
 }
 
 
+// Blocks across a 3D march along y (1) or z (2).
+inline unsigned march_blocks(const Geo &G, int dim)
+{
+    return (unsigned)(((long)(G.NX - 6) * ((dim == 1 ? G.NZ : G.NY) - 6) + 255) / 256);
+}
+
 // Whether the 2D y march is the last sweep (RK combination, closed-form 4x4
 // Newton, Limit and rate inside the march; the separate pass gives the same
 // bits).
@@ -744,7 +756,7 @@ void launch_stage(hipStream_t s, const SweepArgs &a, const double dxs[3], void (
             ay.seg_len = a.seg_y;
             int nseg = (G.NY - 6 + a.seg_y - 1) / a.seg_y;
             timer(tctx, 1, 0);
-            hipLaunchKernelGGL((k_march<5, 1, R, REC, RIEM, false>), dim3(nxb, (G.NZ - 6 + 3) / 4, nseg), dim3(256), 0, s, ay);
+            hipLaunchKernelGGL((k_march<5, 1, R, REC, RIEM, false>), dim3(march_blocks(G, 1), 1, nseg), dim3(256), 0, s, ay);
             timer(tctx, 1, 1);
         }
         {
@@ -753,7 +765,7 @@ void launch_stage(hipStream_t s, const SweepArgs &a, const double dxs[3], void (
             az.seg_len = a.seg_z;
             int nseg = (G.NZ - 6 + a.seg_z - 1) / a.seg_z;
             timer(tctx, 2, 0);
-            hipLaunchKernelGGL((k_march<5, 2, R, REC, RIEM, true>), dim3(nxb, (G.NY - 6 + 3) / 4, nseg), dim3(256), 0, s, az);
+            hipLaunchKernelGGL((k_march<5, 2, R, REC, RIEM, true>), dim3(march_blocks(G, 2), 1, nseg), dim3(256), 0, s, az);
             timer(tctx, 2, 1);
         }
         {
