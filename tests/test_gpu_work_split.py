@@ -189,3 +189,32 @@ def test_x_inside_the_2d_march(shape, kind, rec, riemann, form):
             outs.append((dev.download("P"), dev.download("U")))
     for a, b in zip(*outs):
         assert np.array_equal(a, b, equal_nan=True)
+
+
+@pytest.mark.parametrize("form", ["fp64", "fp64fast"])
+@pytest.mark.parametrize("shape,rec,kind", [((129, 12), "wenoz", "periodic"), ((130, 7), "ppm", "outflow"),
+                                            ((129, 9, 6), "ppm", "outflow"), ((130, 6, 5), "wenoz", "periodic"),
+                                            ((131, 5, 7), "minmod", "outflow")])
+def test_x_march_with_a_narrow_last_wave(shape, rec, kind, form):
+    """x inside the y march where the last wave of a row is one to three
+    columns wide: the stencils of the wave before it reach ghost columns that
+    no pass has written, and have to see the boundary rule's values."""
+    from verona_amd import DeviceGrid
+    progress(f"narrow last wave {shape} {rec} {kind} {form}")
+    nd = len(shape)
+    P = (state2 if nd == 2 else state3)(*shape, seed=11)
+    bc = (kind,) * (2 * nd) + ("none",) * (6 - 2 * nd)
+    outs = []
+    for on in (True, False):
+        with DeviceGrid(nd, *shape, gamma=G) as dev:
+            dev.set_xy_fusion(on)
+            dev.upload("P", P)
+            dev.fill_ghosts(bc)
+            dev.prim_to_cons()
+            dev.set_step(ref_mode=False, rec=rec, riemann="hllc", integrator="rk3", precision=form, n_iter=50, tol=1e-10,
+                         floor=1e-7, cfl=0.3, bc=bc, **{k: 1 / n for k, n in zip(("dx", "dy", "dz"), shape)})
+            for _ in range(3):
+                dev.step()
+            outs.append((dev.download("P"), dev.download("U")))
+    for a, b in zip(*outs):
+        assert np.array_equal(a, b, equal_nan=True)

@@ -331,8 +331,9 @@ __device__ __forceinline__ void edge_faces(const SweepArgs &a, const Geo &G, dou
     const long rb0 = gidx(G, cc, rr, o);
     const long ps = G.ps;
     const R g = (R)a.g, fl = (R)a.floor_;
-    // wave-uniform: only the waves at the x ends of the grid read ghost columns
-    const bool mapx = (a.xmap_lo | a.xmap_hi) != 0 && (x0 == 3 || xr == G.NX - 3);
+    // wave-uniform: only waves within two cells of the x ends read ghost columns
+    // (the face at xr reads cell xr + 2: a ghost too if the next wave is 1 or 2 wide)
+    const bool mapx = (a.xmap_lo | a.xmap_hi) != 0 && (x0 == 3 || xr >= G.NX - 5);
     R q5[5][NV];
     if (mapx) {
         const long row = rb0 - cc;
