@@ -194,11 +194,17 @@ def test_x_inside_the_2d_march(shape, kind, rec, riemann, form):
 @pytest.mark.parametrize("form", ["fp64", "fp64fast"])
 @pytest.mark.parametrize("shape,rec,kind", [((129, 12), "wenoz", "periodic"), ((130, 7), "ppm", "outflow"),
                                             ((129, 9, 6), "ppm", "outflow"), ((130, 6, 5), "wenoz", "periodic"),
-                                            ((131, 5, 7), "minmod", "outflow")])
+                                            ((131, 5, 7), "minmod", "outflow"), ((4, 5, 9), "wenoz", "periodic"),
+                                            ((20, 7, 6), "ppm", "outflow"), ((21, 9, 13), "wenoz", "outflow"),
+                                            ((22, 17, 11), "ppm", "periodic"), ((31, 6, 10), "minmod", "none"),
+                                            ((33, 12, 9), "wenoz", "none"), ((62, 5, 5), "ppm", "outflow"),
+                                            ((63, 8, 7), "wenoz", "periodic"), ((64, 9, 6), "ppm", "periodic"),
+                                            ((65, 7, 9), "minmod", "outflow"), ((97, 10, 8), "wenoz", "outflow")])
 def test_x_march_with_a_narrow_last_wave(shape, rec, kind, form):
-    """x inside the y march where the last wave of a row is one to three
-    columns wide: the stencils of the wave before it reach ghost columns that
-    no pass has written, and have to see the boundary rule's values."""
+    """x inside the y march gives the bits of its own sweep, ghost cells
+    included, where a wave holds the ends of one to four rows and where only
+    one to three columns of a row are left for it: the wave before then reads
+    ghost columns that no pass has written by the boundary rule."""
     from verona_amd import DeviceGrid
     progress(f"narrow last wave {shape} {rec} {kind} {form}")
     nd = len(shape)

@@ -752,11 +752,10 @@ static void partition_sweeps(vrn_ctx *c)
         if (c->xseg > 1) c->rows_per_wave = 1;
     }
     for (int f = 0; f < 2; f++) {
-        // the x-y march (FP64) takes rows of 64 cells, the others any 256 columns
-        const int nxb = (Nxi + 63) / 64;
+        // the FP64 y march is the x-y march
         c->seg_y[f] = march_segment(c->ndim, f == 1, Nyi,
-                                    c->ndim == 2 ? nxb : (f ? (int)march_blocks(c->G, 1) : nxb * ((Nzi + 3) / 4)));
-        if (c->ndim == 3) c->seg_z[f] = march_segment(3, f == 1, Nzi, (int)march_blocks(c->G, 2));
+                                    c->ndim == 3 ? (int)march_blocks(c->G, 1, f == 0) : (Nxi + 63) / 64);
+        if (c->ndim == 3) c->seg_z[f] = march_segment(3, f == 1, Nzi, (int)march_blocks(c->G, 2, false));
     }
 }
 

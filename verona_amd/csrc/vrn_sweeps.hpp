@@ -305,35 +305,47 @@ __global__ __launch_bounds__(256, (xsweep_waves<R, REC>())) void k_xsweep(SweepA
         if (a.do_rate) rate_reduce(a.st, rate);
 }
 
-// ------------------------------------------------------------ x-y march: wave-edge faces
-// The six x faces of rows r0 .. r1-1 at the ends of one wave's 64 columns
-// [x0, x0 + 64) whose stencils leave those columns: faces between cells
-// m - 1 and m for m = x0, x0 + 1, x0 + 2 (edge faces 0..2) and m = xr - 2,
-// xr - 1, xr with xr = min(x0 + 64, NX - 3) (edge faces 3..5).  Lane L
-// reconstructs cell x0 - 1 + i (i = L % 8 < 4) or xr - 3 + (i - 4) of row
-// r0 + L / 8, as the x sweep does (both faces, floors), and lanes with i != 0, 4
-// solve the face with their left neighbour's upper state (DPP shift):
-// exactly the x sweep's faces.  Faces of rows outside [r0, r1) or whose
-// stencil leaves the grid are not needed and not written.  Stencil cells in
-// ghost columns are read through the x boundary rules (xmap_lo / xmap_hi)
-// when the last ghost pass left the x faces unfilled, which gives the values
-// that pass would have written.  Out: ebw[(row - rb) & 7 row stride
-// ebs][face][var].
+// ------------------------------------------------------------ x-y march: edge faces
+// A wave's 64 columns are one or more pieces of rows of cells (nsw of them,
+// the first from column xs of row o0, the last to column xl).  Each piece
+// [x0, xr) has six x faces whose stencils leave it: between cells m - 1 and m
+// for m = x0, x0 + 1, x0 + 2 (edge faces 0..2) and m = xr - 2, xr - 1, xr (edge
+// faces 3..5).  The wave solves them for march rows r0 .. r1-1 at once, eight
+// lanes a piece and row: EdgeMap says how many pieces share a row's lanes and
+// for how many rows there are lanes.  Lane i of eight reconstructs cell
+// x0 - 1 + i (i < 4) or xr - 3 + (i - 4), as the x sweep does (both faces,
+// floors), and lanes with i != 0, 4 solve the face with their left neighbour's
+// upper state (DPP shift): exactly the x sweep's faces.  Faces of rows outside
+// [r0, r1) or whose stencil leaves the grid are not needed and not written.
+// Stencil cells in ghost columns are read through the x boundary rules
+// (xmap_lo / xmap_hi) when the last ghost pass left the x faces unfilled, which
+// gives the values that pass would have written.
+struct EdgeMap {
+    int xs, xl, o0, nsw;
+    int sh;  // log2 of the places for pieces in a row's lanes
+    __device__ __forceinline__ int rows() const { return 8 >> sh; }
+    // place of the first piece of march row r in the edge-face buffer (the
+    // other pieces' follow); 0 where the buffer is to be filled again
+    __device__ __forceinline__ int place(int r) const { return (r << sh) & 7; }
+};
+
 template <int NV, class R, int REC, int RIEM>
-__device__ __forceinline__ void edge_faces(const SweepArgs &a, const Geo &G, double *ebw, int ebs, int lane, int x0,
-                                           int xr, int o, int r0, int r1, int rb)
+__device__ __forceinline__ void edge_faces(const SweepArgs &a, const Geo &G, const EdgeMap &em, double *ebw, int lane,
+                                           int r0, int r1, int rb)
 {
-    const int i = lane & 7, r = r0 + (lane >> 3);
+    const int i = lane & 7, q = lane >> 3;
+    const int r = r0 + (q >> em.sh), seg = q & ((1 << em.sh) - 1);
+    const int x0 = seg == 0 ? em.xs : 3, xr = seg == em.nsw - 1 ? em.xl + 1 : G.NX - 3;
     const int cell = i < 4 ? x0 - 1 + i : xr - 7 + i;
-    const bool ok = r < r1 && cell >= 2 && cell <= G.NX - 3;
+    const bool ok = r < r1 && seg < em.nsw && cell >= 2 && cell <= G.NX - 3;
     const int cc = ok ? cell : 3;
     const int rr = ok ? r : 3;
+    const int o = NV == 5 ? em.o0 + (ok ? seg : 0) : 0;
     const long rb0 = gidx(G, cc, rr, o);
     const long ps = G.ps;
     const R g = (R)a.g, fl = (R)a.floor_;
     // wave-uniform: only waves within two cells of the x ends read ghost columns
-    // (the face at xr reads cell xr + 2: a ghost too if the next wave is 1 or 2 wide)
-    const bool mapx = (a.xmap_lo | a.xmap_hi) != 0 && (x0 == 3 || xr >= G.NX - 5);
+    const bool mapx = (a.xmap_lo | a.xmap_hi) != 0 && (em.nsw > 1 || em.xs <= 5 || em.xl >= G.NX - 6);
     R q5[5][NV];
     if (mapx) {
         const long row = rb0 - cc;
@@ -367,7 +379,7 @@ __device__ __forceinline__ void edge_faces(const SweepArgs &a, const Geo &G, dou
     const bool okl = ok && i != 0 && i != 4 && cell - 3 >= 0;
     if (okl) {
         const int e = i < 4 ? i - 1 : i - 2;
-        double *w = ebw + ((r - rb) & 7) * ebs + e * NV;
+        double *w = ebw + ((em.place(r - rb) + seg) * 6 + e) * NV;
 #pragma unroll
         for (int v = 0; v < NV; v++) w[v] = (double)Ff[v];
     }
@@ -386,14 +398,16 @@ __global__ __launch_bounds__(256, VRN_MARCH_MIN_WAVES) void k_march(SweepArgs a)
     constexpr int WS = NV == 5 ? 256 : 64;
     // XY (y march only): the march also does the x direction of each row
     // it updates, with the ring row of its 64 columns as the x stencils.  The
-    // six faces at a wave's ends whose stencils leave those columns (three
-    // each side) are solved every 8 rows for the next 8 by the whole wave
-    // (edge_faces) into eb[row & 7][wave][face][var].
+    // six faces at a piece's ends whose stencils leave it (three each side)
+    // are solved some rows ahead by the whole wave (edge_faces) into eb, a
+    // region of 8 places a wave.
     static_assert(!XY || (DIM == 1 && (NV == 4 || !LAST)), "x-y fusion is the y march");
     constexpr int WSR = WS;  // ring stride per (slot, variable)
-    __shared__ R win[5 * NV * WSR];
-    constexpr int EBR = (WS / 64) * 6 * NV;  // edge-face buffer stride per row
-    __shared__ double eb[XY ? 8 * EBR : 1];
+    // (the x stencils of the first and last lanes read two words past the ring)
+    __shared__ R win_[5 * NV * WSR + 4];
+    R *const win = win_ + 2;
+    constexpr int EBW = 8 * 6 * NV;  // edge-face buffer of a wave
+    __shared__ double eb[XY ? (WS / 64) * EBW : 1];
     // WENO-Z: the curvature term of each cell (wz_curv) is computed once and
     // carried: cell c needs the terms of cells c-1, c and c+1, and the term of
     // cell x lives in slot x & 1 of a two-slot ring [slot][var][lane].
@@ -407,24 +421,24 @@ __global__ __launch_bounds__(256, VRN_MARCH_MIN_WAVES) void k_march(SweepArgs a)
     const int tid = threadIdx.x;
     const int Nd = DIM == 1 ? G.NY : G.NZ;
     const int No = NV == 5 ? (DIM == 1 ? G.NZ : G.NY) : 7;
-    // the block's columns: 256 consecutive ones of all (x, o), x fastest, so
-    // that only the last block has idle lanes whatever the width (161 cells by
-    // rows of 64 idle 16 % of them); the x-y march needs whole rows of 64
-    constexpr bool PACK = NV == 5 && !XY;
-    const unsigned pt = blockIdx.x * 256 + threadIdx.x, pr = PACK ? pt / (unsigned)(G.NX - 6) : 0;
-    const int x = PACK ? 3 + (int)(pt - pr * (unsigned)(G.NX - 6)) : 3 + blockIdx.x * 64 + (threadIdx.x & 63);
-    int o = PACK ? 3 + (int)pr : 3 + blockIdx.y * (blockDim.x >> 6) + (threadIdx.x >> 6);
+    // the block's columns: consecutive ones of all (x, o), x fastest, so that
+    // only the last block has idle lanes whatever the width (161 cells by rows
+    // of 64 idle 16 % of them; there the x-y march went from 459 to 428 us at
+    // 210 x 99 rows, at 48 x 37 x 29 from 25.5 to 20.8, and at widths of
+    // whole waves, 128 and 384, nothing changed).  a.packw: columns a row takes, the row's cells
+    // or, in the x-y march, 64 where they are few (a wave has places for 4
+    // pieces of rows); one row in 2D
+    const unsigned total = (unsigned)a.packw * (NV == 5 ? No - 6 : 1);
+    const unsigned pt = blockIdx.x * blockDim.x + threadIdx.x, pr = NV == 5 ? pt / (unsigned)a.packw : 0;
+    const int x = 3 + (int)(pt - pr * (unsigned)a.packw);
+    int o = 3 + (int)pr;
     const int m0 = 3 + blockIdx.z * a.seg_len;
     // whole-wave exits only: a partially active wave keeps all lanes for the
     // cross-lane reductions and masks the inactive ones.
-    const bool act = PACK ? o < No - 3 : x < G.NX - 3;
-    if ((PACK ? !__any(act) : o >= No - 3) || m0 >= Nd - 3) return;
-    if (PACK && !act) o = 3;
-    // XY: every lane holds its own column (inactive lanes a ghost or the
-    // last one), since the x stencils of the active lanes reach into them;
-    // ghost columns through the x boundary rules when the last ghost pass
-    // left the x faces unfilled
-    const int xx = XY ? map_coord(min(x, G.NX - 1), G.NX, a.xmap_lo, a.xmap_hi) : (act ? x : 3);
+    const bool act = pt < total && x < G.NX - 3;
+    if (!__any(act) || m0 >= Nd - 3) return;
+    if (!act) o = 3;
+    const int xx = act ? x : 3;
     const int m1 = min(m0 + a.seg_len, Nd - 3);
     const long sd = DIM == 1 ? (long)G.px : (long)G.px * G.NY;
     const long cb = DIM == 1 ? gidx(G, xx, 0, NV == 5 ? o : 0) : gidx(G, xx, o, 0);
@@ -461,14 +475,29 @@ __global__ __launch_bounds__(256, VRN_MARCH_MIN_WAVES) void k_march(SweepArgs a)
             pif[v] = ppm_iface(wl[(0 * NV + v) * WSR], wl[(1 * NV + v) * WSR], wl[(2 * NV + v) * WSR],
                                wl[(3 * NV + v) * WSR]);
     }
+    // XY: the wave's pieces of rows, this lane's piece, the edge face that is
+    // its left face (-1: solved in the wave) and whether its right face is one
     const int wv = tid >> 6;
-    // XY: the edge face that is this lane's left face (-1: solved in the
-    // wave): lanes 0..2 -> edge faces 0..2; lanes 62, 63 -> the right edge's
-    // face at their column (x0 + lane relative to the edge xr = min(x0 + 64,
-    // NX - 3)); lane 63 also takes its right face, edge face 5
-    const int x0 = 3 + blockIdx.x * 64;
-    const int xr = min(x0 + 64, G.NX - 3);
-    const int lfe = lane < 3 ? lane : (lane >= 62 ? 3 + min(max(x0 + lane - xr + 2, 0), 2) : -1);
+    EdgeMap em{};
+    int seg = 0, lfe = -1;
+    bool rfe = false;
+    if constexpr (XY) {
+        const unsigned w0 = __builtin_amdgcn_readfirstlane(pt - lane), wl_ = min(w0 + 63, total - 1);
+        const unsigned q0 = NV == 5 ? w0 / (unsigned)a.packw : 0, q1 = NV == 5 ? wl_ / (unsigned)a.packw : 0;
+        em.xs = 3 + (int)(w0 - q0 * (unsigned)a.packw);
+        em.xl = min(3 + (int)(wl_ - q1 * (unsigned)a.packw), G.NX - 4);
+        em.o0 = 3 + (int)q0;
+        em.nsw = (int)(q1 - q0) + 1;
+        em.sh = em.nsw == 1 ? 0 : (em.nsw == 2 ? 1 : 2);
+        if (act) {
+            seg = (int)(pr - q0);
+            const int d0 = x - (seg == 0 ? em.xs : 3), d1 = (seg == em.nsw - 1 ? em.xl : G.NX - 4) - x;
+            lfe = d0 < 3 ? d0 : (d1 < 2 ? 4 - d1 : -1);
+            rfe = d1 == 0;
+        }
+    }
+    const double *const el = eb + (XY ? wv * EBW + (seg * 6 + max(lfe, 0)) * NV : 0);
+    const double *const er = eb + (XY ? wv * EBW + (seg * 6 + 5) * NV : 0);
     const double cdtx = XY ? (PRE ? a.b : 1.0) * (((a.dt_dev ? a.st->dt : a.dt_fixed) * a.dtfac) / a.dx_x) : 0.0;
     R upp[NV];
     double Fp[NV];
@@ -547,10 +576,10 @@ __global__ __launch_bounds__(256, VRN_MARCH_MIN_WAVES) void k_march(SweepArgs a)
 #pragma unroll
                         for (int v = 0; v < NV; v++) ub[v] = rk_base(a.a, u0b[v], a.b, ub[v]);
                     }
-                    // every 8 rows: the edge faces of rows c-1 .. c+6
-                    if (((c - 1 - m0) & 7) == 0) {
-                        edge_faces<NV, R, REC, RIEM>(a, G, eb + wv * 6 * NV, EBR, lane, x0, xr, NV == 5 ? o : 0, c - 1,
-                                                     min(c + 7, m1), m0);
+                    // the edge faces of this row and the next ones there are
+                    // places for
+                    if (em.place(c - 1 - m0) == 0) {
+                        edge_faces<NV, R, REC, RIEM>(a, G, em, eb + wv * EBW, lane, c - 1, min(c - 1 + em.rows(), m1), m0);
                         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
                         __builtin_amdgcn_wave_barrier();
                         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -583,15 +612,14 @@ __global__ __launch_bounds__(256, VRN_MARCH_MIN_WAVES) void k_march(SweepArgs a)
                     for (int v = 0; v < NV; v++) uplx[v] = shift_up1(upx[v], upx[v]);
                     R Fxf[NV];
                     face_flux<NV, 0, RIEM>(uplx, lox, g, Fxf);
-                    // edge faces of row c-1: each lane reads its own (lfe)
-                    // and edge face 5 (lane 63's right face)
-                    const double *be = eb + ((c - 1 - m0) & 7) * EBR + wv * 6 * NV;
-                    const int lf = lfe < 0 ? 0 : lfe;
+                    // edge faces of row c-1: each lane reads its own (lfe) and
+                    // edge face 5 (the right face of a piece's last lane)
+                    const double *bl = el + em.place(c - 1 - m0) * 6 * NV, *br = er + em.place(c - 1 - m0) * 6 * NV;
 #pragma unroll
                     for (int v = 0; v < NV; v++) {
-                        const double fxl = lfe >= 0 ? be[lf * NV + v] : (double)Fxf[v];
+                        const double fxl = lfe >= 0 ? bl[v] : (double)Fxf[v];
                         const double fxs = shift_down1(fxl, fxl);
-                        const double fxr = lane == 63 ? be[5 * NV + v] : fxs;
+                        const double fxr = rfe ? br[v] : fxs;
                         ub[v] = ub[v] - cdtx * (fxr - fxl);
                     }
                 }
@@ -694,10 +722,13 @@ __global__ __launch_bounds__(64) void k_rescue(SweepArgs a)
 }
 
 
-// Blocks across a 3D march along y (1) or z (2).
-inline unsigned march_blocks(const Geo &G, int dim)
+// Columns that a row of cells takes in a march (SweepArgs::packw) and blocks
+// across a 3D march along y (1) or z (2); xy: the x-y march, whose waves hold
+// at most 4 pieces of rows, so at least 21 columns a row.
+inline int march_width(const Geo &G, bool d3, bool xy) { return d3 && xy && G.NX - 6 < 21 ? 64 : G.NX - 6; }
+inline unsigned march_blocks(const Geo &G, int dim, bool xy)
 {
-    return (unsigned)(((long)(G.NX - 6) * ((dim == 1 ? G.NZ : G.NY) - 6) + 255) / 256);
+    return (unsigned)(((long)march_width(G, true, xy) * ((dim == 1 ? G.NZ : G.NY) - 6) + 255) / 256);
 }
 
 // Whether the 2D y march is the last sweep (RK combination, closed-form 4x4
@@ -732,9 +763,10 @@ void launch_stage(hipStream_t s, const SweepArgs &a, const double dxs[3], void (
             ay.dx_x = dxs[0];
             ay.seg_len = a.seg_y;
             const int nseg = (G.NY - 6 + a.seg_y - 1) / a.seg_y;
+            ay.packw = march_width(G, NV == 5, true);
             timer(tctx, 10, 0);
             if constexpr (NV == 5)
-                hipLaunchKernelGGL((k_march<5, 1, R, REC, RIEM, false, true>), dim3(nxb, (G.NZ - 6 + 3) / 4, nseg),
+                hipLaunchKernelGGL((k_march<5, 1, R, REC, RIEM, false, true>), dim3(march_blocks(G, 1, true), 1, nseg),
                                    dim3(256), 0, s, ay);
             else
                 hipLaunchKernelGGL((k_march<4, 1, R, REC, RIEM, fused_end2d<R>(), true>), dim3(nxb, 1, nseg), dim3(64), 0,
@@ -755,18 +787,20 @@ void launch_stage(hipStream_t s, const SweepArgs &a, const double dxs[3], void (
             SweepArgs ay = a;
             ay.dx_dim = dxs[1];
             ay.seg_len = a.seg_y;
+            ay.packw = march_width(G, true, false);
             int nseg = (G.NY - 6 + a.seg_y - 1) / a.seg_y;
             timer(tctx, 1, 0);
-            hipLaunchKernelGGL((k_march<5, 1, R, REC, RIEM, false>), dim3(march_blocks(G, 1), 1, nseg), dim3(256), 0, s, ay);
+            hipLaunchKernelGGL((k_march<5, 1, R, REC, RIEM, false>), dim3(march_blocks(G, 1, false), 1, nseg), dim3(256), 0, s, ay);
             timer(tctx, 1, 1);
         }
         {
             SweepArgs az = a;
             az.dx_dim = dxs[2];
             az.seg_len = a.seg_z;
+            az.packw = march_width(G, true, false);
             int nseg = (G.NZ - 6 + a.seg_z - 1) / a.seg_z;
             timer(tctx, 2, 0);
-            hipLaunchKernelGGL((k_march<5, 2, R, REC, RIEM, true>), dim3(march_blocks(G, 2), 1, nseg), dim3(256), 0, s, az);
+            hipLaunchKernelGGL((k_march<5, 2, R, REC, RIEM, true>), dim3(march_blocks(G, 2, false), 1, nseg), dim3(256), 0, s, az);
             timer(tctx, 2, 1);
         }
         {
@@ -779,6 +813,7 @@ void launch_stage(hipStream_t s, const SweepArgs &a, const double dxs[3], void (
             SweepArgs ay = a;
             ay.dx_dim = dxs[1];
             ay.seg_len = a.seg_y;
+            ay.packw = march_width(G, false, false);
             timer(tctx, 1, 0);
             hipLaunchKernelGGL((k_march<4, 1, R, REC, RIEM, fused_end2d<R>()>),
                                dim3(nxb, 1, (G.NY - 6 + a.seg_y - 1) / a.seg_y), dim3(64), 0, s, ay);

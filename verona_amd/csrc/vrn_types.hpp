@@ -64,6 +64,7 @@ struct SweepArgs {
     int do_rate;
     int seg_y, seg_z;   // y / z sweeps: interior cells per marching segment
     int seg_len;        // of this march
+    int packw;          // columns that a row of cells takes in this march
     int rows_per_wave;  // x sweep: rows streamed by one wave (xseg == 1)
     int xseg;           // x sweep: segments per row (> 1 only with rows_per_wave == 1)
     // 3D fast FP64 form, x and y directions in one march (0: separate x
