@@ -224,3 +224,27 @@ def test_x_march_with_a_narrow_last_wave(shape, rec, kind, form):
             outs.append((dev.download("P"), dev.download("U")))
     for a, b in zip(*outs):
         assert np.array_equal(a, b, equal_nan=True)
+
+
+@pytest.mark.parametrize("shape", [(660, 7, 620), (700, 50, 8), (330, 8, 311)])
+def test_segments_of_wide_grids(shape):
+    """Grids of so many columns that a march's segments are the fixed ones
+    (also cut to a short axis): the bits of short segments."""
+    from verona_amd import DeviceGrid
+    progress(f"wide grid {shape}")
+    P = state3(*shape, seed=3)
+    bc = ("outflow",) * 6
+    outs = []
+    for seg in (None, 8):
+        with DeviceGrid(3, *shape, gamma=G) as dev:
+            if seg:
+                rows, xseg, _ = dev.partition()
+                dev.set_partition(rows, xseg, seg)
+            dev.upload("P", P)
+            dev.fill_ghosts(bc)
+            dev.prim_to_cons()
+            dev.set_step(ref_mode=False, rec="minmod", riemann="hll", integrator="rk2", precision="fp64fast", n_iter=50,
+                         tol=1e-10, floor=1e-7, cfl=0.3, bc=bc, **{k: 1 / n for k, n in zip(("dx", "dy", "dz"), shape)})
+            dev.step()
+            outs.append(dev.download("P"))
+    assert np.array_equal(*outs, equal_nan=True)

@@ -10,15 +10,17 @@
 //
 // Two kernel sets:
 //  * the reference boundary (vrn_fluxes / vrn_update / vrn_cons_to_prim /
-//    vrn_limit / vrn_prim_to_cons): one thread per face or cell, same
+//    vrn_limit / vrn_prim_to_cons): one lane per face or cell, same
 //    arrays and regions as the Julia KA kernels they replace;
 //  * the fused step (vrn_step): per RK stage, one directional sweep kernel
-//    per axis.  The x sweep runs 64 lanes along a row as a continuous stream
-//    of cells over many rows and passes the upper face state and the face
-//    flux to the next lane with a cross-lane shift; the y and z sweeps give
-//    each lane one (x, .) column and march along the axis with the 5-cell
-//    reconstruction window held in an LDS ring (5 slots x NV variables per
-//    lane, so advancing the window moves no data).  Either way each cell's
+//    per axis, or, in the FP64 forms, one for x and y and one for z.  The x
+//    sweep runs 64 lanes along a row as a continuous stream of cells over many
+//    rows and passes the upper face state and the face flux to the next lane
+//    with a cross-lane shift; the y and z sweeps give each lane one (x, .)
+//    column and march along the axis with the 5-cell reconstruction window
+//    held in an LDS ring (5 slots x NV variables per lane, so advancing the
+//    window moves no data); the x-y march also takes the x direction of each
+//    row from that ring.  Either way each cell's
 //    reconstruction and each face's Riemann solve run exactly once, and all
 //    global loads and stores are row-contiguous across the wave.  The last
 //    sweep of a stage also forms the RK combination, runs 1DW con2prim +
@@ -706,10 +708,20 @@ static int settle(vrn_ctx *c)
 // 48 / 24 / 8 cells 957 / 945 / 961 / 1051 us; 2D 256^2 24 cells 77 us, 1
 // cell 17 us; 2048^2 32 cells 173 us, 24 cells 188 us, 8 cells 177 us.
 // Segments are evened out (the shortest ones of the same count).
+// Large 3D grids, three rounds of blocks or more: 96 cells, or 48 where 96 give
+// fewer rounds.  The model is too coarse there: blocks are so many that the
+// rounds dissolve, and a shorter last segment, dispatched last, fills the end
+// (x-y + z march, us: 256^3, even segments of 32 970 + 683, 64 960 + 680, 96
+// 953 + 678, 48 945 + 667; 320^3 64 1905 + 1326, 48 1894 + 1312, 96 1861 + 1288;
+// 384^3 64 3343 + 2295, 48 3272 + 2257, 96 3270 + 2257; but 224^3, under three
+// rounds of either, 48 695 + 470, 25 678 + 465).
 static int march_segment(int ndim, bool fp32, int L, int cols)
 {
     const int one = 256 * (ndim == 3 ? 1 : 4);  // blocks at one wave per SIMD
     const int slots = one * (fp32 ? 3 : 2);
+    if (ndim == 3)
+        for (int s : {96, 48})
+            if ((long)cols * ((L + s - 1) / s) >= 3 * slots) return std::min(s, L);
     int best = L;
     double least = 1e300;
     for (int n = 1; n <= L && n <= 65535; n++) {
