@@ -15,7 +15,10 @@
 // a tube inside one workgroup; tubes are independent, so no grid-wide
 // synchronisation is needed.  Within a tube the workgroup streams over the
 // cells in chunks of blockDim cells, one cell per lane, exchanging face
-// states and fluxes through LDS with a carry across chunks.
+// states and fluxes through LDS with a carry across chunks.  Where that leaves
+// most of the GPU idle (few tubes, or a few long ones), ranges of the tubes
+// run in workgroups of their own, several steps a launch, with halos wide
+// enough for these steps (k_tubes_split; split_plan chooses).
 //
 // This file holds the C ABI and the exact-form kernels; the kernels
 // themselves are in vrn_tubes_kern.hpp, compiled again as the fast FP64 form

@@ -144,8 +144,9 @@ class DeviceGrid:
               "vrn_set_partition")
 
     def set_xy_fusion(self, on=True):
-        """3D fast FP64 form: x direction inside the y march (default) or as
-        its own sweep; the same arithmetic either way."""
+        """FP64 forms: x direction inside the y march (default; in 2D not for
+        the exact form with PPM and minmod) or as its own sweep; the same
+        arithmetic either way."""
         check(self.lib.vrn_set_xy_fusion(self.h, int(bool(on))), "vrn_set_xy_fusion")
 
     def partition(self):

@@ -4,12 +4,14 @@
     tb.upload(rho, u, ux, dt, dx)           # concatenated SoA, per-tube dt/dx
     tb.set_method("ppm", "hllc", n_iter=50, tol=1e-10)
     shape = tb.autotune()                   # picks (block, grid) on the real data
-    ms = tb.run(500, *shape)                # one persistent hipGraph launch
+    ms = tb.run(500, *shape)                # one launch (or a few, of ranges of tubes)
     rho, u, ux = tb.download()
 
 The launch shape (threads per workgroup, persistent workgroups) is chosen by
 `autotune`, which times each candidate on a checkpointed copy of the actual
-state and caches the winner per (device, problem signature).
+state and caches the winner per (device, problem signature).  Batches too few
+or too uneven to fill the GPU one workgroup a tube run as ranges of tubes with
+overlapping halos instead, in launches whose shape the library chooses.
 """
 import ctypes as C
 import hashlib
