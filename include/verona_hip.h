@@ -236,6 +236,14 @@ int vrn_tubes_set_precision(vrn_tubes *tb, int precision);
  * (the same bits), in launches whose shape the library chooses.
  * *ms receives the device time.  Blocks. */
 int vrn_tubes_run(vrn_tubes *tb, int nsteps, int block, int grid, int use_graph, double *ms);
+/* Whether batches may be run in ranges of tubes (on = 1, the default) or
+ * always as whole tubes, in the launch shape that vrn_tubes_run is given (0);
+ * the same bits either way. */
+int vrn_tubes_set_split(vrn_tubes *tb, int on);
+/* How vrn_tubes_run advances this batch by nsteps steps: in launches of
+ * *launch_steps steps (the last one of what is left) over *ranges ranges of
+ * tubes, its block, grid and use_graph unused; or as whole tubes (0 and 0). */
+int vrn_tubes_plan(vrn_tubes *tb, int nsteps, int *launch_steps, int *ranges);
 /* restore = 0 saves (P, U), restore = 1 puts them back (used by the autotuner). */
 int vrn_tubes_checkpoint(vrn_tubes *tb, int restore);
 int vrn_tubes_info(vrn_tubes *tb, int64_t *ncell, int *cu_count);

@@ -1,0 +1,94 @@
+"""Batched tubes: whole tubes by persistent workgroups in the caller's launch
+shape, and ranges of tubes with halos, each known to be the path that ran."""
+import numpy as np
+import pytest
+
+from helpers import progress
+from test_gpu_tubes import _oracle_tubes
+
+pytestmark = pytest.mark.gpu
+G1 = 5.0 / 3.0
+
+
+def _batch():
+    from verona_amd.tubes import shock_tube_batch
+    return shock_tube_batch(48, lmin=40, lmax=700, seed=7)
+
+
+@pytest.mark.parametrize("rec", ["minmod", "ppm", "wenoz"])
+@pytest.mark.parametrize("riemann", ["hll", "hllc"])
+def test_whole_tubes_in_every_form_and_shape(oracle, rec, riemann):
+    """Whole tubes, eager and replayed graphs, in several launch shapes: the
+    exact form gives the oracle's bits, the fast form the bits of its ranges
+    and the oracle's values to 1e-12 relative L1 where both stay finite."""
+    from verona_amd.tubes import Tubes
+    progress(f"whole tubes {rec} {riemann}")
+    lengths, rho, u, ux, dt, dx = _batch()
+    O = _oracle_tubes(oracle, lengths, rho, u, ux, dt, dx, G1, rec, riemann, 24)
+    with Tubes(lengths) as tb:
+        tb.set_method(rec, riemann, 50, 1e-10)
+        assert tb.plan(24)[0] > 0 and tb.plan(24)[1] > len(lengths)
+        tb.set_precision("fp64fast")
+        tb.upload(rho, u, ux, dt, dx)
+        tb.run(24)
+        F = np.stack(tb.download())
+        tb.set_split(False)
+        assert tb.plan(24) == (0, 0)
+        # a graph of one shape, captured and replayed, in both forms
+        for block, grid, graph in [(64, 1, False), (128, 16, True), (128, 16, False), (1024, 3, False), (256, 48, True)]:
+            for prec, want in (("fp64fast", F), ("fp64", O)):
+                tb.set_precision(prec)
+                tb.upload(rho, u, ux, dt, dx)
+                for _ in range(3):
+                    tb.run(8, block, grid, use_graph=graph)
+                assert np.array_equal(np.stack(tb.download()), want, equal_nan=True), (block, grid, graph, prec)
+    off = np.concatenate([[0], np.cumsum(lengths)])
+    fin = lambda X: np.array([np.isfinite(X[:, off[t]:off[t + 1]]).all() for t in range(len(lengths))])
+    both = fin(O) & fin(F)
+    m = np.repeat(both, lengths)
+    assert both.sum() >= 0.9 * fin(O).sum()
+    for v in range(3):
+        assert np.abs(F[v][m] - O[v][m]).sum() <= 1e-12 * np.abs(O[v][m]).sum()
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp64fast"])
+def test_ranges_and_whole_tubes_in_turn(prec):
+    """Ranges swap the state buffers at each launch: a captured graph of whole
+    tubes before and after them works on the current state."""
+    from verona_amd.tubes import Tubes
+    progress(f"ranges and whole tubes in turn {prec}")
+    lengths, rho, u, ux, dt, dx = _batch()
+    outs = []
+    for turn in (False, True):
+        with Tubes(lengths) as tb:
+            tb.set_method("wenoz", "hllc", 50, 1e-10)
+            tb.set_precision(prec)
+            tb.upload(rho, u, ux, dt, dx)
+            for k in range(9):
+                tb.set_split(turn and k % 3 == 1)
+                assert (tb.plan(4)[0] > 0) == (turn and k % 3 == 1)
+                tb.run(4, 128, 16, use_graph=turn)
+            outs.append(np.stack(tb.download()))
+    assert np.array_equal(*outs, equal_nan=True)
+
+
+def test_batches_left_whole(oracle):
+    """Batches that fill the GPU one workgroup a tube are run whole without
+    being told to."""
+    from verona_amd.tubes import Tubes, shock_tube_batch
+    progress("batches left whole")
+    for n, lo, hi in ((4096, 256, 8192), (1280, 500, 500), (10000, 100, 300)):
+        lengths, rho, u, ux, dt, dx = shock_tube_batch(n, lo, hi, seed=42)
+        with Tubes(lengths) as tb:
+            assert tb.plan(8) == (0, 0), (n, lo, hi)
+            if n != 1280:
+                continue
+            tb.set_method("ppm", "hllc", 50, 1e-10)
+            tb.upload(rho, u, ux, dt, dx)
+            for _ in range(2):
+                tb.run(4, 256, 1024, use_graph=True)
+            G = np.stack(tb.download())
+            for t in (0, 1, 640, 1279):
+                c = slice(500 * t, 500 * (t + 1))
+                O = _oracle_tubes(oracle, [500], rho[c], u[c], ux[c], dt[t:t + 1], dx[t:t + 1], G1, "ppm", "hllc", 8)
+                assert np.array_equal(G[:, c], O, equal_nan=True), t

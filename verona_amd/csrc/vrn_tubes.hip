@@ -81,9 +81,12 @@ struct vrn_tubes {
     hipGraphExec_t gexec = nullptr;
     hipGraph_t graph = nullptr;
     int g_block = 0, g_grid = 0, g_steps = 0, g_rec = -1, g_riem = -1, g_prec = -1;
+    const double *g_state = nullptr;  // the state buffer it works on
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     float last_ms = 0.f;
-    // k_tubes_split: steps a launch (0: whole tubes by k_tubes) and ranges
+    // k_tubes_split: whether it may be used, steps a launch (0: whole tubes by
+    // k_tubes) and ranges
+    bool split = true;
     int split_k = 0, nseg = 0;
     TubeSeg *seg = nullptr;
     double *Psave[3] = {nullptr, nullptr, nullptr}, *Usave[3] = {nullptr, nullptr, nullptr};
@@ -290,12 +293,18 @@ static void launch_tubes(vrn_tubes *c, int block, int grid)
         vrn::launch_tubes_kernels(c->s, c->args, c->rec, c->riemann, block, grid);
 }
 
-// nsteps steps by k_tubes_split, split_k steps a launch (all of them where
-// every tube lies in one workgroup).  The two state buffers change places at
-// each launch.
+// Whether c's tubes are run in ranges (vrn_tubes_set_split, split_plan).
+static bool in_ranges(const vrn_tubes *c) { return c->split && c->split_k; }
+
+// Steps of the launches of nsteps steps in ranges: all of them where every
+// tube lies in one workgroup, else as many as the halos are wide for.
+static int launch_steps(const vrn_tubes *c, int nsteps) { return c->nseg == c->ntubes ? nsteps : std::min(c->split_k, nsteps); }
+
+// nsteps steps by k_tubes_split.  The two state buffers change places at each
+// launch.
 static int run_split(vrn_tubes *c, int nsteps)
 {
-    const int most = c->nseg == c->ntubes ? std::max(nsteps, 1) : c->split_k;
+    const int most = launch_steps(c, nsteps);
     for (int done = 0; done < nsteps;) {
         TubeArgs &a = c->args;
         a.seg = c->seg;
@@ -319,8 +328,10 @@ static int run_split(vrn_tubes *c, int nsteps)
 }
 
 // Advance every tube by nsteps steps: split over workgroups where split_plan
-// says so, else with `grid` persistent workgroups of `block` threads.  use_graph != 0 captures (queue reset + persistent kernel)
-// into a hipGraph once per (block, grid, nsteps, method, precision) and replays it.
+// says so (and vrn_tubes_set_split lets it), else with `grid` persistent
+// workgroups of `block` threads.  use_graph != 0 captures (queue reset +
+// persistent kernel) into a hipGraph once per (block, grid, nsteps, method,
+// precision, state buffer) and replays it.
 // *ms (may be NULL) receives the device time of the launch.  Blocks.
 int vrn_tubes_run(vrn_tubes *c, int nsteps, int block, int grid, int use_graph, double *ms)
 {
@@ -328,13 +339,14 @@ int vrn_tubes_run(vrn_tubes *c, int nsteps, int block, int grid, int use_graph, 
     if (nsteps < 0 || block < 64 || block > 1024 || (block & 63) || grid < 1)
         return tfail(VRN_E_ARG, "bad launch shape (block %d, grid %d)", block, grid);
     c->args.nsteps = nsteps;
-    if (c->split_k) {
+    if (in_ranges(c)) {
         TCHK(hipEventRecord(c->ev0, c->s));
         if (int r = run_split(c, nsteps)) return r;
         TCHK(hipEventRecord(c->ev1, c->s));
     } else if (use_graph) {
         bool stale = !c->gexec || c->g_block != block || c->g_grid != grid || c->g_steps != nsteps ||
-                     c->g_rec != c->rec || c->g_riem != c->riemann || c->g_prec != c->precision;
+                     c->g_rec != c->rec || c->g_riem != c->riemann || c->g_prec != c->precision ||
+                     c->g_state != c->args.P[0];
         if (stale) {
             if (c->gexec) (void)hipGraphExecDestroy(c->gexec);
             if (c->graph) (void)hipGraphDestroy(c->graph);
@@ -350,6 +362,7 @@ int vrn_tubes_run(vrn_tubes *c, int nsteps, int block, int grid, int use_graph, 
             c->g_rec = c->rec;
             c->g_riem = c->riemann;
             c->g_prec = c->precision;
+            c->g_state = c->args.P[0];
         }
         TCHK(hipEventRecord(c->ev0, c->s));
         TCHK(hipGraphLaunch(c->gexec, c->s));
@@ -365,6 +378,26 @@ int vrn_tubes_run(vrn_tubes *c, int nsteps, int block, int grid, int use_graph, 
     TCHK(hipEventElapsedTime(&t, c->ev0, c->ev1));
     c->last_ms = t;
     if (ms) *ms = t;
+    return 0;
+}
+
+// Whether batches may be run in ranges (1, the default) or always as whole
+// tubes in the caller's launch shape (0).
+int vrn_tubes_set_split(vrn_tubes *c, int on)
+{
+    if (!c) return tfail(VRN_E_ARG, "null");
+    c->split = on != 0;
+    return 0;
+}
+
+// How a run of nsteps steps is launched: the steps of its launches in ranges
+// and the ranges, both 0 for whole tubes.
+int vrn_tubes_plan(vrn_tubes *c, int nsteps, int *steps, int *ranges)
+{
+    if (!c || nsteps < 0) return tfail(VRN_E_ARG, "null argument or negative step count");
+    const bool r = in_ranges(c);
+    if (steps) *steps = r ? launch_steps(c, nsteps) : 0;
+    if (ranges) *ranges = r ? c->nseg : 0;
     return 0;
 }
 

@@ -11,7 +11,8 @@ The launch shape (threads per workgroup, persistent workgroups) is chosen by
 `autotune`, which times each candidate on a checkpointed copy of the actual
 state and caches the winner per (device, problem signature).  Batches too few
 or too uneven to fill the GPU one workgroup a tube run as ranges of tubes with
-overlapping halos instead, in launches whose shape the library chooses.
+overlapping halos instead, in launches whose shape the library chooses
+(`plan` says which; `set_split(False)` keeps to whole tubes).
 """
 import ctypes as C
 import hashlib
@@ -36,6 +37,8 @@ TUBE_SIGNATURES = {
     "vrn_tubes_set_method": (_I, [_P, _I, _I, _I, _D]),
     "vrn_tubes_set_precision": (_I, [_P, _I]),
     "vrn_tubes_run": (_I, [_P, _I, _I, _I, _I, _lib._DP]),
+    "vrn_tubes_set_split": (_I, [_P, _I]),
+    "vrn_tubes_plan": (_I, [_P, _I, C.POINTER(_I), C.POINTER(_I)]),
     "vrn_tubes_checkpoint": (_I, [_P, _I]),
     "vrn_tubes_info": (_I, [_P, C.POINTER(C.c_int64), C.POINTER(_I)]),
 }
@@ -127,6 +130,18 @@ class Tubes:
         _check(self.lib.vrn_tubes_run(self.h, int(nsteps), int(block), int(grid), int(bool(use_graph)),
                                       C.byref(ms)), "vrn_tubes_run")
         return ms.value
+
+    def set_split(self, on=True):
+        """Whether the batch may run in ranges of tubes (the default) or always
+        as whole tubes in the launch shape of `run`; the same bits."""
+        _check(self.lib.vrn_tubes_set_split(self.h, int(bool(on))), "vrn_tubes_set_split")
+
+    def plan(self, nsteps):
+        """How run(nsteps) is launched: (steps a launch, ranges of tubes), or
+        (0, 0) for whole tubes."""
+        k, n = _I(), _I()
+        _check(self.lib.vrn_tubes_plan(self.h, int(nsteps), C.byref(k), C.byref(n)), "vrn_tubes_plan")
+        return k.value, n.value
 
     # ------------------------------------------------------------------ autotuner
     def signature(self):
