@@ -92,3 +92,25 @@ def test_batches_left_whole(oracle):
                 c = slice(500 * t, 500 * (t + 1))
                 O = _oracle_tubes(oracle, [500], rho[c], u[c], ux[c], dt[t:t + 1], dx[t:t + 1], G1, "ppm", "hllc", 8)
                 assert np.array_equal(G[:, c], O, equal_nan=True), t
+
+
+def test_autotune_only_where_there_is_a_shape_to_choose(tmp_path):
+    """A batch run in ranges takes no launch shape: autotune times nothing and
+    leaves nothing in its caches; kept whole, the same batch is tuned."""
+    import json
+
+    from verona_amd import tubes
+    from verona_amd.tubes import Tubes
+    progress("autotune and ranges")
+    lengths, rho, u, ux, dt, dx = _batch()
+    f = tmp_path / "shapes.json"
+    with Tubes(lengths, gamma=1.61) as tb:
+        tb.upload(rho, u, ux, dt, dx)
+        tb.set_method("minmod", "hll", 50, 1e-10)
+        shape = tb.autotune(probe_steps=1, cache_file=str(f))
+        assert shape == (128, 2 * tb.cu_count) and tb.autotune_trials == []
+        assert not f.exists() and tb.signature() not in tubes._CACHE
+        tb.set_split(False)
+        shape = tb.autotune(probe_steps=1, cache_file=str(f))
+        assert len(tb.autotune_trials) == len(tubes.BLOCKS) * len(tubes.WAVES_PER_CU)
+        assert tuple(json.loads(f.read_text())[tb.signature()]["shape"]) == shape == tubes._CACHE[tb.signature()]

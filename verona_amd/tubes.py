@@ -123,11 +123,13 @@ class Tubes:
         _check(self.lib.vrn_tubes_set_precision(self.h, codes[precision]), "vrn_tubes_set_precision")
         self.precision = precision
 
+    def _shape(self, block=128, grid=None):
+        return int(block), 2 * self.cu_count if grid is None else int(grid)
+
     def run(self, nsteps, block=128, grid=None, use_graph=True):
-        if grid is None:
-            grid = 2 * self.cu_count
+        block, grid = self._shape(block, grid)
         ms = _D(0.0)
-        _check(self.lib.vrn_tubes_run(self.h, int(nsteps), int(block), int(grid), int(bool(use_graph)),
+        _check(self.lib.vrn_tubes_run(self.h, int(nsteps), block, grid, int(bool(use_graph)),
                                       C.byref(ms)), "vrn_tubes_run")
         return ms.value
 
@@ -153,9 +155,14 @@ class Tubes:
     def autotune(self, probe_steps=2, cache_file=None, verbose=False):
         """Time every (block, workgroups-per-CU) candidate for probe_steps on a
         checkpoint of the current state, restore the state, and return the
-        fastest (block, grid).  Results are cached per problem signature."""
+        fastest (block, grid).  Results are cached per problem signature.  A
+        batch that runs in ranges has no shape to choose: `run`'s default comes
+        back at once and nothing is timed or cached."""
         if self.method is None:
             raise VeronaHIPError("set_method before autotune")
+        if self.plan(probe_steps) != (0, 0):
+            self.autotune_trials = []
+            return self._shape()
         key = self.signature()
         if key in _CACHE:
             return _CACHE[key]
