@@ -114,3 +114,28 @@ def test_autotune_only_where_there_is_a_shape_to_choose(tmp_path):
         shape = tb.autotune(probe_steps=1, cache_file=str(f))
         assert len(tb.autotune_trials) == len(tubes.BLOCKS) * len(tubes.WAVES_PER_CU)
         assert tuple(json.loads(f.read_text())[tb.signature()]["shape"]) == shape == tubes._CACHE[tb.signature()]
+
+
+def test_launches_of_very_many_steps():
+    """Steps a launch stay where the ranges' halo (six cells a step, on both
+    sides of a tube) fits an int, whatever the steps asked for; a run longer
+    than one launch gives the bits of whole tubes."""
+    from verona_amd.tubes import Tubes
+    progress("very many steps")
+    lengths = [40, 62]
+    rng = np.random.default_rng(4)
+    rho, u, ux = (1 + 0.1 * rng.standard_normal(102) for _ in range(3))
+    dx = 1 / np.array(lengths)
+    outs = []
+    for on in (True, False):
+        with Tubes(lengths) as tb:
+            tb.set_split(on)
+            for n in (1, 4097, 2**31 - 1):
+                k, ranges = tb.plan(n)
+                assert (k > 0) == on and k <= n and 6 * k + max(lengths) < 2**31
+            assert ranges == (2 if on else 0)
+            tb.set_method("minmod", "hll", 50, 1e-10)
+            tb.upload(rho, u, ux, 0.1 * dx, dx)
+            tb.run(5000)
+            outs.append(np.stack(tb.download()))
+    assert np.isfinite(outs[0]).all() and np.array_equal(*outs)

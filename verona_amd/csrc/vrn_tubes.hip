@@ -96,6 +96,7 @@ namespace {
 
 constexpr int SPLIT_BLOCK = 256;
 constexpr int SPLIT_CELLS = 62 * (SPLIT_BLOCK / 64);
+constexpr int SPLIT_STEPS = 4096;
 
 // Ranges for k_tubes_split at k steps a launch (tubes that fit a workgroup
 // whole need no halo); the cells they hold in all, halos included.
@@ -296,9 +297,14 @@ static void launch_tubes(vrn_tubes *c, int block, int grid)
 // Whether c's tubes are run in ranges (vrn_tubes_set_split, split_plan).
 static bool in_ranges(const vrn_tubes *c) { return c->split && c->split_k; }
 
-// Steps of the launches of nsteps steps in ranges: all of them where every
-// tube lies in one workgroup, else as many as the halos are wide for.
-static int launch_steps(const vrn_tubes *c, int nsteps) { return c->nseg == c->ntubes ? nsteps : std::min(c->split_k, nsteps); }
+// Steps of the launches of nsteps steps in ranges: as many as the halos are
+// wide for, or, where every tube lies in one workgroup and needs none, up to
+// SPLIT_STEPS (the kernel's halo, 6 cells a step, stays far inside an int, and
+// a launch of 30 ms or more makes its 3 us nothing).
+static int launch_steps(const vrn_tubes *c, int nsteps)
+{
+    return std::min(c->nseg == c->ntubes ? SPLIT_STEPS : c->split_k, nsteps);
+}
 
 // nsteps steps by k_tubes_split.  The two state buffers change places at each
 // launch.
