@@ -139,3 +139,24 @@ def test_launches_of_very_many_steps():
             tb.run(5000)
             outs.append(np.stack(tb.download()))
     assert np.isfinite(outs[0]).all() and np.array_equal(*outs)
+
+
+@pytest.mark.parametrize("change", [dict(n_iter=1), dict(tol=1e-2)])
+def test_graph_of_another_iteration_limit(change):
+    """A captured graph holds the con2prim limit and tolerance it was captured
+    with: other ones need another graph."""
+    from verona_amd.tubes import Tubes
+    progress(f"graph after {change}")
+    lengths, rho, u, ux, dt, dx = _batch()
+    outs = []
+    with Tubes(lengths) as tb:
+        tb.set_split(False)
+        for graph in (True, False):
+            for kw in ({}, change):
+                tb.set_method("ppm", "hllc", **{"n_iter": 50, "tol": 1e-10, **kw})
+                tb.upload(rho, u, ux, dt, dx)
+                tb.run(6, 128, 16, use_graph=graph)
+                outs.append(np.stack(tb.download()))
+    assert np.array_equal(outs[0], outs[2], equal_nan=True)
+    assert np.array_equal(outs[1], outs[3], equal_nan=True)
+    assert not np.array_equal(outs[0], outs[1], equal_nan=True)

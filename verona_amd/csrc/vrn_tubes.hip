@@ -35,6 +35,7 @@
 #include <cstring>
 #include <numeric>
 #include <string>
+#include <tuple>
 #include <vector>
 
 // fast FP64 form of the tube kernels (vrn_tubes_fast.hip)
@@ -80,8 +81,9 @@ struct vrn_tubes {
     // captured graph
     hipGraphExec_t gexec = nullptr;
     hipGraph_t graph = nullptr;
-    int g_block = 0, g_grid = 0, g_steps = 0, g_rec = -1, g_riem = -1, g_prec = -1;
-    const double *g_state = nullptr;  // the state buffer it works on
+    // what it was captured with: launch shape, steps, method (con2prim limits
+    // among it), precision and state buffer
+    std::tuple<int, int, int, int, int, int, double, int, const double *> g_key{};
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     float last_ms = 0.f;
     // k_tubes_split: whether it may be used, steps a launch (0: whole tubes by
@@ -336,8 +338,7 @@ static int run_split(vrn_tubes *c, int nsteps)
 // Advance every tube by nsteps steps: split over workgroups where split_plan
 // says so (and vrn_tubes_set_split lets it), else with `grid` persistent
 // workgroups of `block` threads.  use_graph != 0 captures (queue reset +
-// persistent kernel) into a hipGraph once per (block, grid, nsteps, method,
-// precision, state buffer) and replays it.
+// persistent kernel) into a hipGraph once per g_key and replays it.
 // *ms (may be NULL) receives the device time of the launch.  Blocks.
 int vrn_tubes_run(vrn_tubes *c, int nsteps, int block, int grid, int use_graph, double *ms)
 {
@@ -350,9 +351,9 @@ int vrn_tubes_run(vrn_tubes *c, int nsteps, int block, int grid, int use_graph, 
         if (int r = run_split(c, nsteps)) return r;
         TCHK(hipEventRecord(c->ev1, c->s));
     } else if (use_graph) {
-        bool stale = !c->gexec || c->g_block != block || c->g_grid != grid || c->g_steps != nsteps ||
-                     c->g_rec != c->rec || c->g_riem != c->riemann || c->g_prec != c->precision ||
-                     c->g_state != c->args.P[0];
+        const decltype(c->g_key) key{block, grid, nsteps, c->rec, c->riemann, c->args.n_iter, c->args.tol, c->precision,
+                                     c->args.P[0]};
+        const bool stale = !c->gexec || c->g_key != key;
         if (stale) {
             if (c->gexec) (void)hipGraphExecDestroy(c->gexec);
             if (c->graph) (void)hipGraphDestroy(c->graph);
@@ -362,13 +363,7 @@ int vrn_tubes_run(vrn_tubes *c, int nsteps, int block, int grid, int use_graph, 
             launch_tubes(c, block, grid);
             TCHK(hipStreamEndCapture(c->s, &c->graph));
             TCHK(hipGraphInstantiate(&c->gexec, c->graph, nullptr, nullptr, 0));
-            c->g_block = block;
-            c->g_grid = grid;
-            c->g_steps = nsteps;
-            c->g_rec = c->rec;
-            c->g_riem = c->riemann;
-            c->g_prec = c->precision;
-            c->g_state = c->args.P[0];
+            c->g_key = key;
         }
         TCHK(hipEventRecord(c->ev0, c->s));
         TCHK(hipGraphLaunch(c->gexec, c->s));
