@@ -232,18 +232,20 @@ int vrn_tubes_set_precision(vrn_tubes *tb, int precision);
 /* Advance all tubes by nsteps midpoint-RK2 steps with `grid` persistent
  * workgroups of `block` threads (multiple of 64); use_graph replays a
  * captured hipGraph.  Batches of tubes too few or too uneven to fill the GPU
- * that way are split into ranges of tubes with overlapping halos instead
+ * that way (vrn_tubes_plan) are split into ranges of tubes with overlapping halos instead
  * (the same bits), in launches whose shape the library chooses.
  * *ms receives the device time.  Blocks. */
 int vrn_tubes_run(vrn_tubes *tb, int nsteps, int block, int grid, int use_graph, double *ms);
-/* Whether batches may be run in ranges of tubes (on = 1, the default) or
- * always as whole tubes, in the launch shape that vrn_tubes_run is given (0);
- * the same bits either way. */
-int vrn_tubes_set_split(vrn_tubes *tb, int on);
-/* How vrn_tubes_run advances this batch by nsteps steps: in launches of
- * *launch_steps steps (the last one of what is left) over *ranges ranges of
- * tubes, its block, grid and use_graph unused; or as whole tubes (0 and 0). */
-int vrn_tubes_plan(vrn_tubes *tb, int nsteps, int *launch_steps, int *ranges);
+/* Whether batches are run in ranges of tubes: mode 0 never, 1 (the default)
+ * where that is estimated to be faster than whole tubes in the launch shape
+ * that vrn_tubes_run is given, 2 for every batch that the library would run in
+ * ranges in some launch shape; the same bits. */
+int vrn_tubes_set_split(vrn_tubes *tb, int mode);
+/* How vrn_tubes_run advances this batch by nsteps steps in this launch shape:
+ * in launches of *launch_steps steps (the last one of what is left) over
+ * *ranges ranges of tubes, block, grid and use_graph unused; or as whole tubes
+ * (0 and 0). */
+int vrn_tubes_plan(vrn_tubes *tb, int nsteps, int block, int grid, int *launch_steps, int *ranges);
 /* restore = 0 saves (P, U), restore = 1 puts them back (used by the autotuner). */
 int vrn_tubes_checkpoint(vrn_tubes *tb, int restore);
 int vrn_tubes_info(vrn_tubes *tb, int64_t *ncell, int *cu_count);

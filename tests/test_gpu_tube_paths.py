@@ -27,6 +27,7 @@ def test_whole_tubes_in_every_form_and_shape(oracle, rec, riemann):
     O = _oracle_tubes(oracle, lengths, rho, u, ux, dt, dx, G1, rec, riemann, 24)
     with Tubes(lengths) as tb:
         tb.set_method(rec, riemann, 50, 1e-10)
+        tb.set_split("always")
         assert tb.plan(24)[0] > 0 and tb.plan(24)[1] > len(lengths)
         tb.set_precision("fp64fast")
         tb.upload(rho, u, ux, dt, dx)
@@ -65,7 +66,7 @@ def test_ranges_and_whole_tubes_in_turn(prec):
             tb.set_precision(prec)
             tb.upload(rho, u, ux, dt, dx)
             for k in range(9):
-                tb.set_split(turn and k % 3 == 1)
+                tb.set_split("always" if turn and k % 3 == 1 else False)
                 assert (tb.plan(4)[0] > 0) == (turn and k % 3 == 1)
                 tb.run(4, 128, 16, use_graph=turn)
             outs.append(np.stack(tb.download()))
@@ -94,26 +95,71 @@ def test_batches_left_whole(oracle):
                 assert np.array_equal(G[:, c], O, equal_nan=True), t
 
 
-def test_autotune_only_where_there_is_a_shape_to_choose(tmp_path):
-    """A batch run in ranges takes no launch shape: autotune times nothing and
-    leaves nothing in its caches; kept whole, the same batch is tuned."""
+def test_autotune_measures_ranges_too(tmp_path):
+    """autotune times ranges beside the launch shapes of whole tubes, sets the
+    handle to the faster, also from its caches, and leaves the state alone; a
+    handle kept to one path is tuned in that path alone."""
     import json
 
     from verona_amd import tubes
-    from verona_amd.tubes import Tubes
+    from verona_amd.tubes import Tubes, shock_tube_batch
     progress("autotune and ranges")
-    lengths, rho, u, ux, dt, dx = _batch()
+    shapes = len(tubes.BLOCKS) * len(tubes.WAVES_PER_CU)
     f = tmp_path / "shapes.json"
-    with Tubes(lengths, gamma=1.61) as tb:
-        tb.upload(rho, u, ux, dt, dx)
+    for n, L, ranges_win in ((2, 8000, True), (256, 1000, False)):
+        lengths, rho, u, ux, dt, dx = shock_tube_batch(n, L, L, seed=3)
+        outs = []
+        for repeat in (0, 1, 2):
+            with Tubes(lengths, gamma=1.61) as tb:
+                tb.upload(rho, u, ux, dt, dx)
+                tb.set_method("minmod", "hll", 50, 1e-10)
+                if repeat == 2:
+                    tubes._CACHE.clear()  # leaves the file
+                shape = tb.autotune(probe_steps=1, cache_file=str(f))
+                key = tb.signature() + ":ranges"
+                if repeat == 0:
+                    assert len(tb.autotune_trials) == shapes + 1
+                    assert tb.autotune_trials[-1][0] < min(tb.autotune_trials[:-1])[0] or not ranges_win
+                    assert json.loads(f.read_text())[key]["shape"] == list(tubes._CACHE[key])
+                assert not hasattr(tb, "autotune_trials") or repeat == 0
+                assert (tubes._CACHE[key] == ()) == (tb.plan(5, *shape) != (0, 0))
+                if ranges_win:
+                    assert tb.plan(5, *shape) != (0, 0) and shape == (128, 2 * tb.cu_count)
+                tb.run(5, *shape)
+                outs.append(np.stack(tb.download()))
+        assert np.array_equal(outs[0], outs[1], equal_nan=True) and np.array_equal(outs[0], outs[2], equal_nan=True)
+    with Tubes([300, 500]) as tb:
         tb.set_method("minmod", "hll", 50, 1e-10)
-        shape = tb.autotune(probe_steps=1, cache_file=str(f))
-        assert shape == (128, 2 * tb.cu_count) and tb.autotune_trials == []
-        assert not f.exists() and tb.signature() not in tubes._CACHE
+        tb.upload(*(np.ones(800),) * 3, 1e-4, 1.0)
+        tb.set_split("always")
+        assert tb.autotune() == (128, 2 * tb.cu_count) and tb.autotune_trials == []
         tb.set_split(False)
-        shape = tb.autotune(probe_steps=1, cache_file=str(f))
-        assert len(tb.autotune_trials) == len(tubes.BLOCKS) * len(tubes.WAVES_PER_CU)
-        assert tuple(json.loads(f.read_text())[tb.signature()]["shape"]) == shape == tubes._CACHE[tb.signature()]
+        tb.autotune(probe_steps=1)
+        assert len(tb.autotune_trials) == shapes and tb.plan(1) == (0, 0)
+
+
+@pytest.mark.parametrize("n,length,shape,ranges", [(512, 500, (512, 512), False), (512, 500, (128, 512), True),
+                                                   (256, 1000, (1024, 256), False), (256, 1000, (128, 512), True),
+                                                   (64, 4000, (1024, 256), True), (1, 3000, (1024, 1), True)])
+def test_ranges_only_where_faster_than_the_given_shape(n, length, shape, ranges):
+    """Whether a batch runs in ranges depends on the launch shape that it is
+    given: the faster path, measured, is the one that runs."""
+    from verona_amd.tubes import Tubes, shock_tube_batch
+    progress(f"{n} tubes of {length} in {shape}")
+    lengths, rho, u, ux, dt, dx = shock_tube_batch(n, length, length, seed=5)
+    with Tubes(lengths) as tb:
+        tb.set_method("ppm", "hllc", 50, 1e-10)
+        assert (tb.plan(32, *shape) != (0, 0)) == ranges
+        ms = {}
+        for mode in ("always", False):
+            tb.set_split(mode)
+            t = []
+            for _ in range(4):
+                tb.upload(rho, u, ux, dt, dx)
+                t.append(tb.run(32, *shape, use_graph=False))
+            ms[mode] = min(t)
+        progress(f"  ranges {ms['always']:.3f} ms, whole tubes {ms[False]:.3f} ms")
+        assert (ms["always"] < ms[False]) == ranges
 
 
 def test_launches_of_very_many_steps():
@@ -129,7 +175,7 @@ def test_launches_of_very_many_steps():
     outs = []
     for on in (True, False):
         with Tubes(lengths) as tb:
-            tb.set_split(on)
+            tb.set_split("always" if on else False)
             for n in (1, 4097, 2**31 - 1):
                 k, ranges = tb.plan(n)
                 assert (k > 0) == on and k <= n and 6 * k + max(lengths) < 2**31

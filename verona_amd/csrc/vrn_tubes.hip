@@ -86,10 +86,14 @@ struct vrn_tubes {
     std::tuple<int, int, int, int, int, int, double, int, const double *> g_key{};
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     float last_ms = 0.f;
-    // k_tubes_split: whether it may be used, steps a launch (0: whole tubes by
-    // k_tubes) and ranges
-    bool split = true;
+    // k_tubes_split: 0 never, 1 where it is the faster, 2 wherever split_plan
+    // has a plan; steps a launch (0: no plan) and ranges
+    int split = 1;
     int split_k = 0, nseg = 0;
+    // for ranges_faster: lengths (longest first), their sum, and the time of a
+    // stage in ranges and in whole tubes in the best launch shape
+    std::vector<long> len;
+    double cells = 0.0, t_ranges = 0.0, t_whole = 0.0;
     TubeSeg *seg = nullptr;
     double *Psave[3] = {nullptr, nullptr, nullptr}, *Usave[3] = {nullptr, nullptr, nullptr};
 };
@@ -116,8 +120,9 @@ long split_ranges(const int64_t *lengths, const std::vector<int> &order, int k, 
     return cells;
 }
 
-// How a batch is run: 0 for whole tubes by persistent workgroups (k_tubes),
-// else the steps a launch of k_tubes_split and its ranges.  Persistent
+// The plan for ranges: 0 if a batch is better run as whole tubes by persistent
+// workgroups (k_tubes) in any launch shape, else the steps a launch of
+// k_tubes_split and its ranges.  Persistent
 // workgroups take about 8 us a stage for each 256 cells of the longest tube,
 // and 3.9e-5 us a cell when the chip is full; ranges take at least 6 us a
 // stage, 4.4e-5 us a cell (halos included) and 3 us a launch.  So split
@@ -126,6 +131,7 @@ long split_ranges(const int64_t *lengths, const std::vector<int> &order, int k, 
 // steps, persistent / split: 8 tubes of 1000 to 3000 cells 3.29 / 0.41 ms;
 // 256 of 4000 8.8 / 3.4; 1024 of 256 to 8192 17.2 / 13.3; 2000 of 100 to 700
 // (HLL) 3.15 / 3.40; 1280 of 500 2.22 / 2.87; 4096 of 256 to 8192 43.9 / 50.4.
+// Between, the launch shape decides (ranges_faster).
 int split_plan(int ntubes, const int64_t *lengths, const std::vector<int> &order, std::vector<TubeSeg> &seg)
 {
     long total = 0;
@@ -142,6 +148,63 @@ int split_plan(int ntubes, const int64_t *lengths, const std::vector<int> &order
     }
     if (best) split_ranges(lengths, order, best, &seg);
     return best;
+}
+
+// us a stage in ranges and as whole tubes in the best launch shape, for
+// ranges_faster, of a batch that has a plan
+void stage_times(vrn_tubes *c, const std::vector<TubeSeg> &seg)
+{
+    double waves = 0.0, lanes = 0.0;
+    for (const TubeSeg &g : seg) waves += c->len[0] <= SPLIT_CELLS ? (g.hi - g.lo + 61) / 62 : SPLIT_BLOCK / 64;
+    const double n = (double)seg.size();
+    if (c->len[0] <= SPLIT_CELLS)  // no halo, all steps in a launch
+        c->t_ranges = n <= 1280 ? 0.0065 * c->cells / SPLIT_CELLS : 0.0035 * n + 0.00075 * waves;
+    else
+        c->t_ranges = 0.0035 * n + 0.00075 * waves + 2.1 / c->split_k;
+    c->t_ranges = std::max(4.4, 3.6 + c->t_ranges);
+    auto face_lanes = [&](size_t t) { return (double)((c->len[t] + 64) / 64 * 64); };
+    double most = 0.0;
+    for (size_t t = 0; t < c->len.size(); t++) lanes += face_lanes(t);
+    for (size_t j = 0; 256 * j < c->len.size(); j++) most = std::max(most, (j + 1) * face_lanes(256 * j));
+    const bool full = lanes / 256 > most || lanes > 1e6;
+    c->t_whole = std::max(5.9, 2.9 + (full ? 0.0085 : 0.0072) * std::max(most, lanes / 256));
+}
+
+// Whether a batch that has a plan is faster in ranges than as whole tubes by
+// `grid` workgroups of `block` threads.  Times of a stage in us, the geometric
+// mean of both forms and four methods (minmod + HLL, PPM + HLL, PPM + HLLC,
+// WENO-Z + HLLC), measured on 60 batches of 1 to 3000 tubes of 16 to 12000
+// cells:
+//  * ranges take 3.6 + 0.0065 a full workgroup (4.4 at least) and 2.1 for a
+//    launch, which has 2 k stages (standard deviation 8 %);
+//  * whole tubes in the best of 12 shapes take 2.9 + 0.0072 a cell of the
+//    busiest CU, 0.0085 where all CUs are busy or a million cells no longer
+//    fit the L2s, 5.9 at least (8 %);
+//  * in a given shape a workgroup goes through its tubes in chunks of `block`
+//    cells, each 2.8 plus 0.24 for each wave that the CU runs at a time (20 at
+//    most; a batch of few tubes fills some CUs before others) (17 %);
+//  * ranges / whole tubes of a form and reconstruction lies off the mean by
+//    the factors below.
+// Whole tubes in the best shape / ranges: 122 of 390 6.6 / 6.2, 256 of 500 7.4 /
+// 9.0, 512 of 500 10.5 / 13.3, 256 of 1000 10.1 / 12.5, 64 of 1000 9.0 / 6.0, 256
+// of 2000 19 / 21, 400 of 2000 34 / 29; by 512 workgroups of 128 threads ranges
+// win in all of them (512 of 500 19).  Run in ranges whatever the shape, 306 of
+// 5952 runs (496 of a plan, 12 shapes) took 5 to 47 % longer than whole tubes in
+// their shape; by this rule 100 do, 54 of them by more than 10 %, and 58 are whole that
+// ranges would run 5 % faster or more.
+bool ranges_faster(const vrn_tubes *c, int block, int grid)
+{
+    const long n = (long)c->len.size(), w = block / 64, G = std::min<long>(grid, 256 * (20 / w));
+    auto chunks = [&](long t) { return (double)((c->len[t] + block) / block); };
+    double mean = 0.0, most = 0.0;
+    for (long t = 0; t < n; t++) mean += chunks(t) / (double)G;
+    for (long j = 0; G * j < n; j++) most = std::max(most, (j + 1) * chunks(G * j));
+    const double per_cu = std::max(1.0, std::min((double)G / 256, std::max(1.0, (double)n / 128)));
+    const double chunk = 2.8 + 0.24 * per_cu * (double)w * (c->cells > 1e6 ? 1.3 : 1.0);
+    static const double off[3][2] = {{0.98, 0.86}, {1.11, 1.00}, {1.03, 0.94}};  // minmod, PPM, WENO-Z
+    static_assert(VRN_REC_MINMOD == 0 && VRN_REC_PPM == 1 && VRN_REC_WENOZ == 2, "rows of off");
+    const double ranges = c->t_ranges * off[c->rec][c->precision == VRN_PREC_FP64_FAST];
+    return ranges < std::max(c->t_whole, 1.6 + std::max(mean, most) * chunk);
 }
 
 }  // namespace
@@ -171,6 +234,11 @@ int vrn_tubes_create(int ntubes, const int64_t *lengths, double gamma, vrn_tubes
     std::vector<TubeSeg> seg;
     c->split_k = split_plan(ntubes, lengths, order, seg);
     c->nseg = (int)seg.size();
+    if (c->split_k) {
+        for (int t : order) c->len.push_back(lengths[t]);
+        c->cells = (double)total;
+        stage_times(c, seg);
+    }
     // one allocation for the state (P, Ph, U, Uh, P0, Psave, Usave x 3
     // variables) and the tables, the constant ones of which (off, order, seg)
     // are copied together
@@ -296,8 +364,11 @@ static void launch_tubes(vrn_tubes *c, int block, int grid)
         vrn::launch_tubes_kernels(c->s, c->args, c->rec, c->riemann, block, grid);
 }
 
-// Whether c's tubes are run in ranges (vrn_tubes_set_split, split_plan).
-static bool in_ranges(const vrn_tubes *c) { return c->split && c->split_k; }
+// Whether c's tubes are run in ranges when the launch shape is this.
+static bool in_ranges(const vrn_tubes *c, int block, int grid)
+{
+    return c->split_k && c->split && (c->split == 2 || ranges_faster(c, block, grid));
+}
 
 // Steps of the launches of nsteps steps in ranges: as many as the halos are
 // wide for, or, where every tube lies in one workgroup and needs none, up to
@@ -335,18 +406,23 @@ static int run_split(vrn_tubes *c, int nsteps)
     return 0;
 }
 
-// Advance every tube by nsteps steps: split over workgroups where split_plan
-// says so (and vrn_tubes_set_split lets it), else with `grid` persistent
-// workgroups of `block` threads.  use_graph != 0 captures (queue reset +
+static int check_shape(int nsteps, int block, int grid)
+{
+    if (nsteps < 0 || block < 64 || block > 1024 || (block & 63) || grid < 1)
+        return tfail(VRN_E_ARG, "bad launch shape (block %d, grid %d)", block, grid);
+    return 0;
+}
+
+// Advance every tube by nsteps steps: split over workgroups where in_ranges
+// says so, else with `grid` persistent workgroups of `block` threads.  use_graph != 0 captures (queue reset +
 // persistent kernel) into a hipGraph once per g_key and replays it.
 // *ms (may be NULL) receives the device time of the launch.  Blocks.
 int vrn_tubes_run(vrn_tubes *c, int nsteps, int block, int grid, int use_graph, double *ms)
 {
     if (!c || !c->params) return tfail(VRN_E_STATE, "vrn_tubes_set_method first");
-    if (nsteps < 0 || block < 64 || block > 1024 || (block & 63) || grid < 1)
-        return tfail(VRN_E_ARG, "bad launch shape (block %d, grid %d)", block, grid);
+    if (int r = check_shape(nsteps, block, grid)) return r;
     c->args.nsteps = nsteps;
-    if (in_ranges(c)) {
+    if (in_ranges(c, block, grid)) {
         TCHK(hipEventRecord(c->ev0, c->s));
         if (int r = run_split(c, nsteps)) return r;
         TCHK(hipEventRecord(c->ev1, c->s));
@@ -382,21 +458,22 @@ int vrn_tubes_run(vrn_tubes *c, int nsteps, int block, int grid, int use_graph, 
     return 0;
 }
 
-// Whether batches may be run in ranges (1, the default) or always as whole
-// tubes in the caller's launch shape (0).
-int vrn_tubes_set_split(vrn_tubes *c, int on)
+// Whether batches are run in ranges: never (0), where that is the faster (1,
+// the default) or wherever there is a plan for it (2).
+int vrn_tubes_set_split(vrn_tubes *c, int mode)
 {
-    if (!c) return tfail(VRN_E_ARG, "null");
-    c->split = on != 0;
+    if (!c || mode < 0 || mode > 2) return tfail(VRN_E_ARG, "null, or mode outside 0..2");
+    c->split = mode;
     return 0;
 }
 
-// How a run of nsteps steps is launched: the steps of its launches in ranges
-// and the ranges, both 0 for whole tubes.
-int vrn_tubes_plan(vrn_tubes *c, int nsteps, int *steps, int *ranges)
+// How a run of nsteps steps in a launch shape is launched: the steps of its
+// launches in ranges and the ranges, both 0 for whole tubes.
+int vrn_tubes_plan(vrn_tubes *c, int nsteps, int block, int grid, int *steps, int *ranges)
 {
-    if (!c || nsteps < 0) return tfail(VRN_E_ARG, "null argument or negative step count");
-    const bool r = in_ranges(c);
+    if (!c) return tfail(VRN_E_ARG, "null");
+    if (int r = check_shape(nsteps, block, grid)) return r;
+    const bool r = in_ranges(c, block, grid);
     if (steps) *steps = r ? launch_steps(c, nsteps) : 0;
     if (ranges) *ranges = r ? c->nseg : 0;
     return 0;

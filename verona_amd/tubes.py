@@ -11,8 +11,8 @@ The launch shape (threads per workgroup, persistent workgroups) is chosen by
 `autotune`, which times each candidate on a checkpointed copy of the actual
 state and caches the winner per (device, problem signature).  Batches too few
 or too uneven to fill the GPU one workgroup a tube run as ranges of tubes with
-overlapping halos instead, in launches whose shape the library chooses
-(`plan` says which; `set_split(False)` keeps to whole tubes).
+overlapping halos instead where that is faster, in launches whose shape the
+library chooses (`plan` says which, `set_split` decides, `autotune` measures).
 """
 import ctypes as C
 import hashlib
@@ -38,7 +38,7 @@ TUBE_SIGNATURES = {
     "vrn_tubes_set_precision": (_I, [_P, _I]),
     "vrn_tubes_run": (_I, [_P, _I, _I, _I, _I, _lib._DP]),
     "vrn_tubes_set_split": (_I, [_P, _I]),
-    "vrn_tubes_plan": (_I, [_P, _I, C.POINTER(_I), C.POINTER(_I)]),
+    "vrn_tubes_plan": (_I, [_P, _I, _I, _I, C.POINTER(_I), C.POINTER(_I)]),
     "vrn_tubes_checkpoint": (_I, [_P, _I]),
     "vrn_tubes_info": (_I, [_P, C.POINTER(C.c_int64), C.POINTER(_I)]),
 }
@@ -71,6 +71,7 @@ class Tubes:
         self.gamma = float(gamma)
         self.method = None
         self.precision = "fp64"
+        self.split = True
         n = C.c_int64()
         cu = _I()
         _check(self.lib.vrn_tubes_info(self.h, C.byref(n), C.byref(cu)), "vrn_tubes_info")
@@ -134,15 +135,20 @@ class Tubes:
         return ms.value
 
     def set_split(self, on=True):
-        """Whether the batch may run in ranges of tubes (the default) or always
-        as whole tubes in the launch shape of `run`; the same bits."""
-        _check(self.lib.vrn_tubes_set_split(self.h, int(bool(on))), "vrn_tubes_set_split")
+        """Whether the batch runs in ranges of tubes: True (the default) where
+        that is estimated to be faster than whole tubes in the launch shape of
+        `run`, False never, "always" wherever the library has ranges for it;
+        the same bits."""
+        mode = 2 if on == "always" else int(bool(on))
+        _check(self.lib.vrn_tubes_set_split(self.h, mode), "vrn_tubes_set_split")
+        self.split = on
 
-    def plan(self, nsteps):
-        """How run(nsteps) is launched: (steps a launch, ranges of tubes), or
-        (0, 0) for whole tubes."""
+    def plan(self, nsteps, block=128, grid=None):
+        """How run(nsteps, block, grid) is launched: (steps a launch, ranges of
+        tubes), or (0, 0) for whole tubes."""
         k, n = _I(), _I()
-        _check(self.lib.vrn_tubes_plan(self.h, int(nsteps), C.byref(k), C.byref(n)), "vrn_tubes_plan")
+        _check(self.lib.vrn_tubes_plan(self.h, int(nsteps), *self._shape(block, grid), C.byref(k), C.byref(n)),
+               "vrn_tubes_plan")
         return k.value, n.value
 
     # ------------------------------------------------------------------ autotuner
@@ -155,50 +161,73 @@ class Tubes:
     def autotune(self, probe_steps=2, cache_file=None, verbose=False):
         """Time every (block, workgroups-per-CU) candidate for probe_steps on a
         checkpoint of the current state, restore the state, and return the
-        fastest (block, grid).  Results are cached per problem signature.  A
-        batch that runs in ranges has no shape to choose: `run`'s default comes
-        back at once and nothing is timed or cached."""
+        fastest (block, grid).  Results are cached per problem signature.
+
+        Where the batch may also run in ranges of tubes, these are timed too
+        (all for as many steps as a launch of ranges takes, up to 16), and the
+        handle is set to what won: set_split("always"), with `run`'s default
+        shape returned, or set_split(False)."""
         if self.method is None:
             raise VeronaHIPError("set_method before autotune")
-        if self.plan(probe_steps) != (0, 0):
-            self.autotune_trials = []
-            return self._shape()
-        key = self.signature()
-        if key in _CACHE:
-            return _CACHE[key]
-        if cache_file and os.path.exists(cache_file):
+        asked = self.split
+        if asked:
+            self.set_split("always")
+            steps = self.plan(16)[0]
+            if asked == "always" and steps:
+                self.autotune_trials = []
+                return self._shape()
+            if steps:
+                probe_steps = max(probe_steps, steps)
+            else:
+                self.set_split(asked)
+        ranges = asked and steps > 0  # set to run in ranges
+        key = self.signature() + (":ranges" if ranges else "")
+        disk = {}
+        if key not in _CACHE and cache_file and os.path.exists(cache_file):
             try:
                 disk = json.load(open(cache_file))
                 if key in disk:
                     _CACHE[key] = tuple(disk[key]["shape"])
-                    return _CACHE[key]
             except (OSError, ValueError):
-                pass
+                disk = {}
+        if key not in _CACHE:
+            _CACHE[key] = self._time_shapes(ranges, probe_steps, verbose)
+            if cache_file:
+                try:
+                    disk[key] = {"shape": list(_CACHE[key]), "trials": [list(r) for r in self.autotune_trials]}
+                    os.makedirs(os.path.dirname(os.path.abspath(cache_file)), exist_ok=True)
+                    json.dump(disk, open(cache_file, "w"))
+                except (OSError, ValueError):
+                    pass
+        shape = _CACHE[key]
+        if ranges:
+            self.set_split(False if shape else "always")
+        return shape or self._shape()
+
+    def _time_shapes(self, ranges, steps, verbose):
+        """The fastest launch shape of whole tubes; () if ranges of tubes are
+        to be timed too and are faster than all of them."""
+        def time(what, shape):
+            self.run(steps, *shape, use_graph=False)  # warm
+            _check(self.lib.vrn_tubes_checkpoint(self.h, 1), "restore")
+            ms = self.run(steps, *shape, use_graph=False)
+            _check(self.lib.vrn_tubes_checkpoint(self.h, 1), "restore")
+            if verbose:
+                print(f"  autotune {what}: {ms:.3f} ms", flush=True)
+            return (ms, *shape)
+
         _check(self.lib.vrn_tubes_checkpoint(self.h, 0), "checkpoint")
-        results = []
+        in_ranges = time("ranges", self._shape())[0] if ranges else float("inf")
+        if ranges:
+            self.set_split(False)
+        trials = []
         for block in BLOCKS:
             for wpc in WAVES_PER_CU:
                 grid = max(1, (wpc * 64 * self.cu_count) // block)
-                self.run(probe_steps, block, grid, use_graph=False)  # warm
-                _check(self.lib.vrn_tubes_checkpoint(self.h, 1), "restore")
-                ms = self.run(probe_steps, block, grid, use_graph=False)
-                _check(self.lib.vrn_tubes_checkpoint(self.h, 1), "restore")
-                results.append((ms, block, grid))
-                if verbose:
-                    print(f"  autotune block={block} grid={grid}: {ms:.3f} ms", flush=True)
-        best = min(results)
-        shape = (best[1], best[2])
-        _CACHE[key] = shape
-        if cache_file:
-            try:
-                disk = json.load(open(cache_file)) if os.path.exists(cache_file) else {}
-                disk[key] = {"shape": list(shape), "trials": [[r[0], r[1], r[2]] for r in results]}
-                os.makedirs(os.path.dirname(os.path.abspath(cache_file)), exist_ok=True)
-                json.dump(disk, open(cache_file, "w"))
-            except (OSError, ValueError):
-                pass
-        self.autotune_trials = results
-        return shape
+                trials.append(time(f"block={block} grid={grid}", (block, grid)))
+        self.autotune_trials = trials + ([(in_ranges,)] if ranges else [])
+        best = min(trials)
+        return best[1:] if best[0] < in_ranges else ()
 
 
 def shock_tube_batch(ntubes, lmin=256, lmax=8192, seed=42, gamma=5.0 / 3.0):
