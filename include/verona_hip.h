@@ -187,10 +187,11 @@ int vrn_timing_report(vrn_ctx *ctx, char *names, int name_len, int64_t *counts, 
  * changes no arithmetic, every face and cell is computed once either way):
  * x sweep: rows_per_wave whole rows per wavefront, or, with xseg > 1, one of
  * xseg segments of a row per wavefront (then rows_per_wave must be 1);
- * y / z sweeps: seg_len interior cells per marching segment.  vrn_create
- * chooses a partition for the grid, with a segment for each march and form
- * (from 1 cell on small grids); vrn_get_partition reads it back, as seg_len
- * the FP64 y march's and at least 8, the least that can be set. */
+ * y / z sweeps: seg_len interior cells (8 to 4096) per marching segment, or 0:
+ * the segments that vrn_create chooses for this grid, one length for each
+ * march and form (from 1 cell on small grids).  vrn_create chooses the whole
+ * partition, with seg_len 0; vrn_get_partition reads it back in the form that
+ * vrn_set_partition takes. */
 int vrn_set_partition(vrn_ctx *ctx, int rows_per_wave, int xseg, int seg_len);
 int vrn_get_partition(vrn_ctx *ctx, int *rows_per_wave, int *xseg, int *seg_len);
 

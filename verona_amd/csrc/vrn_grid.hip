@@ -520,7 +520,8 @@ struct vrn_ctx {
     double dxs[3] = {1, 1, 1};
     // tuning
     int rows_per_wave = 8;
-    int seg_y[2] = {96, 96}, seg_z[2] = {96, 96};  // FP64, FP32 forms
+    int seg_y[2] = {96, 96}, seg_z[2] = {96, 96};  // chosen for this grid: FP64, FP32 forms
+    int seg_set = 0;                               // set for all marches (0: the chosen ones)
     int xseg = 1;
     // timing
     int timing = 0;  // 0 off, 1 every kernel, 2 the directional sweeps only
@@ -1242,8 +1243,8 @@ int vrn_step(vrn_ctx *c, const vrn_step_params *p, double *dt_used)
     a.dt_fixed = p->dt;
     a.dt_dev = cflm ? 1 : 0;
     const int sf = p->precision == VRN_PREC_FP32 ? 1 : 0;
-    a.seg_y = c->seg_y[sf];
-    a.seg_z = c->seg_z[sf];
+    a.seg_y = c->seg_set ? c->seg_set : c->seg_y[sf];
+    a.seg_z = c->seg_set ? c->seg_set : c->seg_z[sf];
     a.rows_per_wave = c->rows_per_wave;
     a.xseg = c->xseg;
     a.fuse_xy = c->fuse_xy;
@@ -1325,7 +1326,7 @@ int vrn_set_partition(vrn_ctx *c, int rows_per_wave, int xseg, int seg_len)
     if (int r = check_ctx(c)) return r;
     const int Nxi = c->G.NX - 6;
     if (rows_per_wave < 1 || rows_per_wave > 64 || xseg < 1 || (xseg > 1 && rows_per_wave != 1) ||
-        xseg > Nxi || seg_len < 8 || seg_len > 4096)
+        xseg > Nxi || (seg_len != 0 && (seg_len < 8 || seg_len > 4096)))
         return fail(VRN_E_ARG, "bad sweep partition (rows_per_wave %d, xseg %d, seg_len %d)", rows_per_wave,
                     xseg, seg_len);
     // a row segment streams at least 34 cells (x0-1 .. x1 with >= 32 interior
@@ -1334,7 +1335,7 @@ int vrn_set_partition(vrn_ctx *c, int rows_per_wave, int xseg, int seg_len)
         return fail(VRN_E_ARG, "row segments shorter than 32 cells (nx %d, xseg %d)", Nxi, xseg);
     c->rows_per_wave = rows_per_wave;
     c->xseg = xseg;
-    for (int f = 0; f < 2; f++) c->seg_y[f] = c->seg_z[f] = seg_len;
+    c->seg_set = seg_len;
     return 0;
 }
 
@@ -1350,9 +1351,7 @@ int vrn_get_partition(vrn_ctx *c, int *rows_per_wave, int *xseg, int *seg_len)
     if (int r = check_ctx(c)) return r;
     if (rows_per_wave) *rows_per_wave = c->rows_per_wave;
     if (xseg) *xseg = c->xseg;
-    // while each march has its own: the FP64 y march's, at least the least that
-    // vrn_set_partition takes
-    if (seg_len) *seg_len = std::max(8, c->seg_y[0]);
+    if (seg_len) *seg_len = c->seg_set;
     return 0;
 }
 

@@ -140,6 +140,8 @@ class DeviceGrid:
 
     # ------------------------------------------------------------------ work partition
     def set_partition(self, rows_per_wave, xseg, seg_len):
+        """Work partition of the sweeps; seg_len 0: the march segments chosen for
+        the grid (what partition() gives until another length is set)."""
         check(self.lib.vrn_set_partition(self.h, int(rows_per_wave), int(xseg), int(seg_len)),
               "vrn_set_partition")
 
