@@ -74,14 +74,16 @@ bool ready(int dev)
     return true;
 }
 
-bool pinned(const void *host)
+// Whether CPU threads may copy at this address: memory that the runtime knows
+// (pinned, managed, a device's) is left to it.
+bool pageable(const void *host)
 {
     hipPointerAttribute_t a{};
     if (hipPointerGetAttributes(&a, host) != hipSuccess) {
         (void)hipGetLastError();
-        return false;
+        return true;
     }
-    return a.type == hipMemoryTypeHost;
+    return a.type == hipMemoryTypeUnregistered;
 }
 
 // One thread's share of a staged copy: the slices k = t, t + THREADS, ...
@@ -186,14 +188,14 @@ void release()
 hipError_t h2d(void *dev, const void *host, size_t n, hipStream_t s)
 {
     hipError_t e;
-    if (n >= LARGE_UP && !pinned(host) && staged(false, const_cast<void *>(host), dev, n, s, &e)) return e;
+    if (n >= LARGE_UP && pageable(host) && staged(false, const_cast<void *>(host), dev, n, s, &e)) return e;
     return hipMemcpyAsync(dev, host, n, hipMemcpyHostToDevice, s);
 }
 
 hipError_t d2h(void *host, const void *dev, size_t n, hipStream_t s)
 {
     hipError_t e;
-    if (n >= LARGE_DOWN && !pinned(host) && staged(true, host, const_cast<void *>(dev), n, s, &e)) return e;
+    if (n >= LARGE_DOWN && pageable(host) && staged(true, host, const_cast<void *>(dev), n, s, &e)) return e;
     e = hipMemcpyAsync(host, dev, n, hipMemcpyDeviceToHost, s);
     return e == hipSuccess ? hipStreamSynchronize(s) : e;
 }

@@ -3,8 +3,8 @@
 // The runtime moves pageable memory at 29 GB/s to the device and 17 GB/s from
 // it (one thread staging), pinned memory at 57 GB/s both ways.  Large copies
 // therefore go through pinned staging slots here, filled and emptied by a few
-// threads while the link moves the neighbouring slots; small ones, and host
-// arrays that are pinned already, go to the runtime directly.
+// threads while the link moves the neighbouring slots; small ones, and
+// memory that the runtime knows, go to the runtime directly.
 #pragma once
 #include <hip/hip_runtime.h>
 
