@@ -5,8 +5,8 @@
 #include <atomic>
 #include <cstdint>
 #include <cstring>
+#include <exception>
 #include <mutex>
-#include <system_error>
 #include <thread>
 
 namespace {
@@ -124,6 +124,7 @@ hipError_t share(int t, int dev, bool down, char *host, char *device, size_t n, 
     }
     // the slots still on the stream
     for (long i = std::max(0L, used - SLOTS); i < used; i++) finish(i, t + i * THREADS);
+    if (e != hipSuccess) (void)hipStreamSynchronize(s);  // also a copy whose event could not be recorded
     if (e != hipSuccess) failed.store(1, std::memory_order_relaxed);
     return e;
 }
@@ -154,7 +155,7 @@ bool staged(bool down, void *host, void *device, size_t n, hipStream_t s, hipErr
                 e[t] = share(t, dev, down, static_cast<char *>(host), static_cast<char *>(device), n, failed);
             });
             run[t] = true;
-        } catch (const std::system_error &) {  // no thread to be had: the caller takes its share
+        } catch (const std::exception &) {  // no thread or memory to be had: the caller takes its share
         }
     }
     for (int t = 0; t < THREADS; t++)
