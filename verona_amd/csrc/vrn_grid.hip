@@ -493,7 +493,7 @@ struct vrn_ctx {
     double gamma = 4.0 / 3.0;
     double *buf = nullptr;   // P, Pn, U, Uh and the staging buffer
     double *fbuf = nullptr;  // flux slots, allocated by the first per-kernel call that uses them
-    int fuse_xy = 1;  // 3D FP64 forms: x direction inside the y march
+    int fuse_xy = 1;  // FP64 forms: x direction inside the y march where launch_stage has that
     // 3D FP64 forms with the fused x-y march and rules on both x faces:
     // the stage-end ghost passes leave the x faces unfilled (the x-y march,
     // their only reader in the step, reads ghost columns through the rules);

@@ -300,8 +300,9 @@ template <class T> __device__ __forceinline__ void minmod(T qm1, T q, T qp1, T &
 
 // x / 6 in FP64: x (1/6) plus one remainder correction (Markstein: with 1/6
 // rounded to nearest and a first quotient within an ulp, the corrected
-// quotient is the correctly rounded x / 6).  Where the remainder is not exact
-// (0 < |x| < 2^-1010) the exact form divides; v_div_fixup gives +-0, +-inf and
+// quotient is the correctly rounded x / 6).  Where the remainder may be
+// inexact the exact form divides (from 2^-1010 down; the test draws the line at
+// 2^-1000); v_div_fixup gives +-0, +-inf and
 // NaN as the division does.  5 instructions for the division's 11 (FP32: the
 // IEEE division).
 template <class T> __device__ __forceinline__ T div6(T x)

@@ -394,10 +394,10 @@ __device__ __forceinline__ void edge_faces(const SweepArgs &a, const Geo &G, con
 template <int NV, int DIM, class R, int REC, int RIEM, bool LAST, bool XY = false>
 __global__ __launch_bounds__(256, VRN_MARCH_MIN_WAVES) void k_march(SweepArgs a)
 {
-    // lanes per block: 256 in 3D (four o-rows of 64 columns), 64 in 2D
+    // lanes per block, a column each: 256 in 3D, 64 in 2D
     constexpr int WS = NV == 5 ? 256 : 64;
     // XY (y march only): the march also does the x direction of each row
-    // it updates, with the ring row of its 64 columns as the x stencils.  The
+    // it updates, with a wave's 64 words of the ring row as the x stencils.  The
     // six faces at a piece's ends whose stencils leave it (three each side)
     // are solved some rows ahead by the whole wave (edge_faces) into eb, a
     // region of 8 places a wave.
@@ -750,8 +750,9 @@ void launch_stage(hipStream_t s, const SweepArgs &a, const double dxs[3], void (
     // sweep's write and the y sweep's re-read of the accumulated U and one
     // read of P per stage; the same fluxes and updates in the same order as
     // the x and y sweeps.  In 2D the fast form's stage is then one kernel
-    // (fused / split, us a stage: 2048^2 WENO-Z 282 / 300, PPM 364 / 440,
-    // minmod 204 / 241; 512^2 WENO-Z 35 / 51); the exact form gains with
+    // (fused / split, us a stage: 2048^2 WENO-Z 270 / 299, PPM 363 / 435,
+    // minmod 220 / 271, 10 % more for all of them in the first steps; 512^2
+    // WENO-Z 35 / 51); the exact form gains with
     // WENO-Z (1024^2 105 / 129, 2048^2 366 / 377) and not with the others
     // (2048^2 PPM 583 / 546, minmod 244 / 233), whose selects already fill
     // the march.

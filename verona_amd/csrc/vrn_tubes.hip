@@ -18,7 +18,7 @@
 // states and fluxes through LDS with a carry across chunks.  Where that leaves
 // most of the GPU idle (few tubes, or a few long ones), ranges of the tubes
 // run in workgroups of their own, several steps a launch, with halos wide
-// enough for these steps (k_tubes_split; split_plan chooses).
+// enough for these steps (k_tubes_split; split_plan and ranges_faster choose).
 //
 // This file holds the C ABI and the exact-form kernels; the kernels
 // themselves are in vrn_tubes_kern.hpp, compiled again as the fast FP64 form
@@ -122,13 +122,13 @@ long split_ranges(const int64_t *lengths, const std::vector<int> &order, int k, 
 
 // The plan for ranges: 0 if a batch is better run as whole tubes by persistent
 // workgroups (k_tubes) in any launch shape, else the steps a launch of
-// k_tubes_split and its ranges.  Persistent
+// k_tubes_split and its ranges.  Figures of
+// exact PPM + HLLC in workgroups of 128 threads, two a CU: persistent
 // workgroups take about 8 us a stage for each 256 cells of the longest tube,
 // and 3.9e-5 us a cell when the chip is full; ranges take at least 6 us a
 // stage, 4.4e-5 us a cell (halos included) and 3 us a launch.  So split
 // ranges win while tubes are too few or too uneven to fill the chip, and
-// persistent workgroups when it is full.  Measured, exact PPM + HLLC, 32
-// steps, persistent / split: 8 tubes of 1000 to 3000 cells 3.29 / 0.41 ms;
+// persistent workgroups when it is full.  Measured, 32 steps, persistent / split: 8 tubes of 1000 to 3000 cells 3.29 / 0.41 ms;
 // 256 of 4000 8.8 / 3.4; 1024 of 256 to 8192 17.2 / 13.3; 2000 of 100 to 700
 // (HLL) 3.15 / 3.40; 1280 of 500 2.22 / 2.87; 4096 of 256 to 8192 43.9 / 50.4.
 // Between, the launch shape decides (ranges_faster).
@@ -414,9 +414,10 @@ static int check_shape(int nsteps, int block, int grid)
 }
 
 // Advance every tube by nsteps steps: split over workgroups where in_ranges
-// says so, else with `grid` persistent workgroups of `block` threads.  use_graph != 0 captures (queue reset +
-// persistent kernel) into a hipGraph once per g_key and replays it.
-// *ms (may be NULL) receives the device time of the launch.  Blocks.
+// says so, else with `grid` persistent workgroups of `block` threads.
+// use_graph != 0 captures (queue reset + persistent kernel) into a hipGraph once
+// per g_key and replays it.  *ms (may be NULL) receives the device time of the
+// launches.  Blocks.
 int vrn_tubes_run(vrn_tubes *c, int nsteps, int block, int grid, int use_graph, double *ms)
 {
     if (!c || !c->params) return tfail(VRN_E_STATE, "vrn_tubes_set_method first");

@@ -67,8 +67,9 @@ struct SweepArgs {
     int packw;          // columns that a row of cells takes in this march
     int rows_per_wave;  // x sweep: rows streamed by one wave (xseg == 1)
     int xseg;           // x sweep: segments per row (> 1 only with rows_per_wave == 1)
-    // 3D fast FP64 form, x and y directions in one march (0: separate x
-    // sweep, the same results), and the x spacing of its flux differences
+    // FP64 forms: x and y directions in one march where launch_stage has that
+    // (0: separate x sweep, the same results), and the x spacing of its flux
+    // differences
     int fuse_xy;
     double dx_x;
     // x-y march: boundary rules through which its x reads of ghost columns

@@ -1,7 +1,7 @@
 // vrn_xfer.hpp -- copies between pageable host arrays and the device.
 //
-// The runtime moves pageable memory at 29 GB/s to the device and 17 GB/s from
-// it (one thread staging), pinned memory at 57 GB/s both ways.  Large copies
+// The runtime moves pageable memory at 27 to 29 GB/s to the device and 17 GB/s
+// from it (one thread staging), pinned memory at 57 GB/s both ways.  Large copies
 // therefore go through pinned staging slots here, filled and emptied by a few
 // threads while the link moves the neighbouring slots; small ones, and
 // memory that the runtime knows, go to the runtime directly.
