@@ -122,16 +122,16 @@ long split_ranges(const int64_t *lengths, const std::vector<int> &order, int k, 
 
 // The plan for ranges: 0 if a batch is better run as whole tubes by persistent
 // workgroups (k_tubes) in any launch shape, else the steps a launch of
-// k_tubes_split and its ranges.  Figures of
-// exact PPM + HLLC in workgroups of 128 threads, two a CU: persistent
-// workgroups take about 8 us a stage for each 256 cells of the longest tube,
-// and 3.9e-5 us a cell when the chip is full; ranges take at least 6 us a
-// stage, 4.4e-5 us a cell (halos included) and 3 us a launch.  So split
-// ranges win while tubes are too few or too uneven to fill the chip, and
-// persistent workgroups when it is full.  Measured, 32 steps, persistent / split: 8 tubes of 1000 to 3000 cells 3.29 / 0.41 ms;
-// 256 of 4000 8.8 / 3.4; 1024 of 256 to 8192 17.2 / 13.3; 2000 of 100 to 700
-// (HLL) 3.15 / 3.40; 1280 of 500 2.22 / 2.87; 4096 of 256 to 8192 43.9 / 50.4.
-// Between, the launch shape decides (ranges_faster).
+// k_tubes_split and its ranges.  For exact PPM + HLLC: persistent workgroups of
+// 256 threads take about 8 us a stage for each 256 cells of the longest tube,
+// and 3.9e-5 us a cell when the chip is full; ranges take at least 6 us a stage,
+// 4.4e-5 us a cell (halos included) and 3 us a launch.  So ranges win while
+// tubes are too few or too uneven to fill the chip, and persistent workgroups
+// when it is full.  32 steps, persistent / ranges: 8 tubes of 1000 to 3000 cells
+// 3.29 / 0.41 ms; 256 of 4000 8.8 / 3.4; 1024 of 256 to 8192 17.2 / 13.3; 2000 of
+// 100 to 700 (HLL) 3.15 / 3.40; 1280 of 500 2.22 / 2.87; 4096 of 256 to 8192 43.9 /
+// 50.4.  In other launch shapes whole tubes may be the faster where there is a
+// plan too: ranges_faster.
 int split_plan(int ntubes, const int64_t *lengths, const std::vector<int> &order, std::vector<TubeSeg> &seg)
 {
     long total = 0;
