@@ -127,6 +127,11 @@ def test_autotune_measures_ranges_too(tmp_path):
                     assert tb.plan(5, *shape) != (0, 0) and shape == (128, 2 * tb.cu_count)
                 tb.run(5, *shape)
                 outs.append(np.stack(tb.download()))
+                # another method is measured anew, ranges too, whatever won before
+                if repeat == 0:
+                    tb.set_method("ppm", "hllc", 50, 1e-10)
+                    tb.autotune(probe_steps=1)
+                    assert len(tb.autotune_trials) == shapes + 1
         assert np.array_equal(outs[0], outs[1], equal_nan=True) and np.array_equal(outs[0], outs[2], equal_nan=True)
     with Tubes([300, 500]) as tb:
         tb.set_method("minmod", "hll", 50, 1e-10)

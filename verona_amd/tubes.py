@@ -139,9 +139,12 @@ class Tubes:
         that is estimated to be faster than whole tubes in the launch shape of
         `run`, False never, "always" wherever the library has ranges for it;
         the same bits."""
+        self._use(on)
+        self.split = on
+
+    def _use(self, on):
         mode = 2 if on == "always" else int(bool(on))
         _check(self.lib.vrn_tubes_set_split(self.h, mode), "vrn_tubes_set_split")
-        self.split = on
 
     def plan(self, nsteps, block=128, grid=None):
         """How run(nsteps, block, grid) is launched: (steps a launch, ranges of
@@ -165,13 +168,13 @@ class Tubes:
 
         Where the batch may also run in ranges of tubes, these are timed too
         (all for as many steps as a launch of ranges takes, up to 16), and the
-        handle is set to what won: set_split("always"), with `run`'s default
-        shape returned, or set_split(False)."""
+        handle runs what won from then on, until set_split or the next
+        autotune: ranges, with `run`'s default shape returned, or whole tubes."""
         if self.method is None:
             raise VeronaHIPError("set_method before autotune")
         asked = self.split
         if asked:
-            self.set_split("always")
+            self._use("always")
             steps = self.plan(16)[0]
             if asked == "always" and steps:
                 self.autotune_trials = []
@@ -179,7 +182,7 @@ class Tubes:
             if steps:
                 probe_steps = max(probe_steps, steps)
             else:
-                self.set_split(asked)
+                self._use(asked)
         ranges = asked and steps > 0  # set to run in ranges
         key = self.signature() + (":ranges" if ranges else "")
         disk = {}
@@ -201,7 +204,7 @@ class Tubes:
                     pass
         shape = _CACHE[key]
         if ranges:
-            self.set_split(False if shape else "always")
+            self._use(False if shape else "always")
         return shape or self._shape()
 
     def _time_shapes(self, ranges, steps, verbose):
@@ -219,7 +222,7 @@ class Tubes:
         _check(self.lib.vrn_tubes_checkpoint(self.h, 0), "checkpoint")
         in_ranges = time("ranges", self._shape())[0] if ranges else float("inf")
         if ranges:
-            self.set_split(False)
+            self._use(False)
         trials = []
         for block in BLOCKS:
             for wpc in WAVES_PER_CU:
